@@ -77,7 +77,7 @@ struct Side {
   std::array<int, MAXL + 1> nb{};  // host copy of box counts per level
 };
 
-struct M2LLev;  // one level of an M2L launch (kernels.hip)
+struct M2LLev;  // one level of an M2L launch (m2l.h)
 
 struct Engine {
   fmmx_config cfg{};
@@ -230,7 +230,7 @@ struct Engine {
   int build_lists();
   int build_far_lists();
   int build_m2l_order();
-  // kernels.hip
+  // p2p.hip, p2m.hip, l2p.hip, translate.hip, m2l.hip
   int run_p2p(int neq);
   int run_p2m(int neq);
   int run_m2m(int lev);

@@ -1,5 +1,5 @@
 // m2l.h -- expansion layouts, reflection signs and launch descriptors shared
-// by the M2L kernels (kernels.hip: FP32 and FP64 forms; m2l_split.hip: the
+// by the M2L kernels (m2l.hip: FP32 and FP64 forms; m2l_split.hip: the
 // error-compensated FP16 form).
 #pragma once
 

@@ -4,7 +4,7 @@
 // (the hi/lo splitting of Ootomo and Yokota, "Recovering single precision
 // accuracy from Tensor Cores while surpassing the FP32 theoretical peak
 // performance", IJHPCA 2022).  The tiling, class order, offset splits and XCD
-// mapping are those of the FP32 MFMA kernel (kernels.hip, k_m2l): a workgroup
+// mapping are those of the FP32 MFMA kernel (m2l.hip, k_m2l): a workgroup
 // owns a tile of targets of one parity class at a level, all sharing the 189
 // offsets of kernel/m2l.cxx's far list (fmm/ijbox.cxx:366-401); per offset the
 // split operator is staged in LDS and every wave multiplies it with its
