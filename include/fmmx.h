@@ -206,8 +206,10 @@ int fmmx_set_yukawa(fmmx_handle* h, double lambda);
  * register prefetch, 2 double buffer, up to p = 11; 3 and 4: the
  * error-compensated FP16 kernel on 16x16x32 MFMA with one or two operator
  * buffers, 5: the same on 32x32x16 MFMA (32 targets per wave, or 64 with 4
- * N-tiles, p <= 10); FP32 engine, Laplace, EXACT convention, p = 6..12),
- * waves per workgroup (4|8|16, 16 with staging 2), offset splits (1..16); 0
+ * N-tiles, p <= 10); FP32 engine, Laplace, EXACT convention, p = 6..12; 6,
+ * the default of p = 6..10: the sources of reflected offsets combined before
+ * the product, 63 products per target), waves per workgroup (4|8|16, 16 with
+ * staging 2, 8 with staging 6), offset splits (1..16); 0
  * (-1 for staging) keeps the default.  The FP64
  * and Helmholtz kernels use the split count only.  fmmx_get_m2l_variant returns the four
  * values in effect (after set_points).  The tuner that picks them by timing

@@ -194,6 +194,8 @@ struct OpSet {
   int split_e = 0;
   // the same split for the 32x32x16 kernel: all 316 operators as they act
   std::vector<uint4> m2l_wide;
+  // the same split for the reflection-orbit kernel: its NORBOP operators
+  std::vector<uint4> m2l_orbit;
   int nlev = 1;
 };
 std::mutex g_cache_mu;
@@ -302,6 +304,7 @@ std::shared_ptr<OpSet> get_ops(const Tables& T, int lmax, float rd) {
       }
       S->split_e = split_scale_exp(ck.data(), ck.size());
       split_fragments(ck.data(), NCANON, T.p, S->split_e, S->m2l_split);
+      if (m2l_orbit_supported(T.p)) orbit_fragments(S->m2l_kmaj.data(), T.p, S->split_e, S->m2l_orbit);
       if (split_wide_fits(T.p)) split_fragments_wide(S->m2l_kmaj.data(), NOFF, T.p, S->split_e, S->m2l_wide);
     }
   }
@@ -593,6 +596,22 @@ int Engine::init(const fmmx_config* c, int dev, void* strm) {
   }
   if ((rc = offtab_s.ensure(ot.size() * 4))) return rc;
   FMMX_HIP(hipMemcpy(offtab_s.p, ot.data(), ot.size() * 4, hipMemcpyHostToDevice));
+  // reflection orbits of each class: base offset, operator and the sign
+  // combinations of the doubled axes in order (3 bits each)
+  std::vector<int> ob(8 * NORB * 4);
+  for (int cls = 0; cls < 8; cls++)
+    for (int o = 0; o < NORB; o++) {
+      int* e = &ob[((size_t)cls * NORB + o) * 4];
+      orbit_offset(o, cls, e);
+      const int D = orb_mask(o), op = orbit_op_index(e);
+      if (op < 0) return fail(FMMX_ESTATE, "M2L orbit outside the operator table");
+      uint32_t subs = 0;
+      for (int r = 0, k = 0; r < 8; r++)
+        if (!(r & ~D)) subs |= (uint32_t)r << (3 * k++);
+      e[3] = (int)((uint32_t)op | subs << 8);
+    }
+  if ((rc = orbtab.ensure(ob.size() * 4))) return rc;
+  FMMX_HIP(hipMemcpy(orbtab.p, ob.data(), ob.size() * 4, hipMemcpyHostToDevice));
   return FMMX_OK;
 }
 
@@ -684,26 +703,30 @@ int Engine::upload_operators() {
     if ((rc = upload<float>(op_m2m, S->m2m_frag, stream)) || (rc = upload<float>(op_l2l, S->l2l_frag, stream)) ||
         (rc = upload<float>(op_m2l, canon ? S->m2l_canon : S->m2l_frag, stream)))
       return rc;
-    split_ok = false;
-    if (canon && !S->m2l_split.empty()) {
-      if ((rc = op_m2l_h.ensure(S->m2l_split.size() * 16))) return rc;
-      FMMX_HIP(hipMemcpyAsync(op_m2l_h.p, S->m2l_split.data(), S->m2l_split.size() * 16, hipMemcpyHostToDevice,
-                              stream));
-      FMMX_HIP(hipStreamSynchronize(stream));
-      sa_e = S->split_e;
-      split_ok = true;
-    }
-    wide_ok = false;
-    if (split_ok && !S->m2l_wide.empty()) {
-      if ((rc = op_m2l_w.ensure(S->m2l_wide.size() * 16))) return rc;
-      FMMX_HIP(hipMemcpyAsync(op_m2l_w.p, S->m2l_wide.data(), S->m2l_wide.size() * 16, hipMemcpyHostToDevice,
-                              stream));
-      FMMX_HIP(hipStreamSynchronize(stream));
-      wide_ok = true;
-    }
+    // the FP16 forms' operators go up with their first launch (upload_split)
+    split_ok = canon && !S->m2l_split.empty();
+    wide_ok = split_ok && !S->m2l_wide.empty();
+    orb_ok = split_ok && !S->m2l_orbit.empty();
+    sa_e = S->split_e;
+    up_h = up_w = up_o = false;
   }
   ops_lmax = lmax;
   ops_rd = rd;
+  return FMMX_OK;
+}
+
+int Engine::upload_split(int form) {
+  bool& up = form == 6 ? up_o : form == 5 ? up_w : up_h;
+  if (up) return FMMX_OK;
+  if (capturing) return fail(FMMX_ESTATE, "M2L operators not uploaded before capture");
+  auto S = get_ops(tab, ops_lmax, ops_rd);  // built at upload_operators: a lookup
+  const std::vector<uint4>& v = form == 6 ? S->m2l_orbit : form == 5 ? S->m2l_wide : S->m2l_split;
+  DevBuf& dst = form == 6 ? op_m2l_o : form == 5 ? op_m2l_w : op_m2l_h;
+  int rc = dst.ensure(v.size() * 16);
+  if (rc) return rc;
+  FMMX_HIP(hipMemcpyAsync(dst.p, v.data(), v.size() * 16, hipMemcpyHostToDevice, stream));
+  FMMX_HIP(hipStreamSynchronize(stream));
+  up = true;
   return FMMX_OK;
 }
 
@@ -1334,7 +1357,7 @@ int fmmx_set_m2l_variant(fmmx_handle* h, int lev, int nt, int staging, int wpg, 
   FMMX_GUARD({
     if (!h) return fmmx::fail(FMMX_EINVAL, "handle is NULL");
     if (lev < 2 || lev > fmmx::MAXL) return fmmx::fail(FMMX_EINVAL, "level out of range [2, 8]");
-    if (nt < 0 || nt > 4 || nt == 3 || (nt == 4 && staging != 5) || staging < -1 || staging > 5 || (wpg != 0 && wpg != 4 && wpg != 8 && wpg != 16) ||
+    if (nt < 0 || nt > 4 || nt == 3 || (nt == 4 && staging != 5) || staging < -1 || staging > 6 || (wpg != 0 && wpg != 4 && wpg != 8 && wpg != 16) ||
         nsplit < 0 || nsplit > 16)
       return fmmx::fail(FMMX_EINVAL, "bad M2L variant");
     auto& t = h->e.tune[lev];

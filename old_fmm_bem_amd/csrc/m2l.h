@@ -99,6 +99,92 @@ struct WLayout {
 // largest magnitude of the scaled split operands (2^14)
 constexpr int SPLIT_TOP = 14;
 
+// Reflection orbits of the M2L offsets.  T_r (ReflMask) is diagonal, so the
+// real slots fall into 8 classes by their signs under the three reflections:
+// class kappa (bits x, y, z) holds the slots with T_r = (-1)^popcount(kappa & r).
+// The offsets (+-dx, +-dy, +-dz) that one target sees form an orbit, whose
+// sum over the sources s_r at the reflected offsets is
+//   sum_r T_r A T_r s_r:  row class c, column class kappa:  A(c, kappa) S_{c ^ kappa},
+//   S_psi = sum_r (-1)^popcount(psi & r) s_r   (a Walsh-Hadamard transform),
+// one dense product for all of them.  A component of magnitude 0 or 3 appears
+// with one sign only (3 with the sign of the target's parity), so an orbit
+// doubles the axes in a mask D and the transform runs over those.  The seven
+// orbits that double every axis are taken as two halves of either z sign, so
+// that no product has more than 4 sources (registers): 63 products per target
+// instead of 189, numbered by their mask D (orb_start).
+//
+// Storage of a class: member i (in slot order) is word i / 4 of lane group
+// i % 4.  A step of the product takes one word of every class (an octet: 8
+// words per lane, position t = class t); the words that at most four classes
+// have beyond the octets form a last step of four words (a quad).
+constexpr int NORB = 63, ORB_WPG = 8;
+// first product of mask D (D = 7: the end); D = 3 holds its own 7 and the 14
+// halves of the fully doubled orbits
+constexpr __host__ __device__ int orb_start(int D) { return D <= 3 ? 7 * D : 7 * D + 14; }
+constexpr __host__ __device__ int orb_mask(int o) { return o < 21 ? o / 7 : o < 42 ? 3 : o / 7 - 2; }
+constexpr int NORBOP = 124;  // distinct operators over the eight parity classes
+constexpr __host__ __device__ int orb_class(int n, int m, int im) {
+  return ((m ^ im) & 1) | im << 1 | ((n + m) & 1) << 2;
+}
+template <int P>
+struct OLayout {
+  static constexpr int P2 = P * P, RW = 16;  // rows of a class's output tile
+  int size[8];         // slots of a class
+  int16_t slot[8][RW * 2];  // class member -> slot, -1 beyond the class
+  int no;              // octet steps
+  int quad;            // 1: a quad step follows
+  int qc[4];           // classes of the quad step (a class with no word left where fewer than four have one)
+  constexpr OLayout() : size{}, slot{}, no(0), quad(0), qc{} {
+    for (int k = 0; k < 8; k++)
+      for (int i = 0; i < RW * 2; i++) slot[k][i] = -1;
+    int c = 0;
+    for (int im = 0; im < 2; im++)
+      for (int n = 0; n < P; n++)
+        for (int m = im; m <= n; m++, c++) {
+          const int k = orb_class(n, m, im);
+          slot[k][size[k]++] = (int16_t)c;
+        }
+    // the fewest octets that leave words in at most four classes
+    for (no = 0;; no++) {
+      int left = 0, more = 0;
+      for (int k = 0; k < 8; k++) {
+        if (size[k] > 4 * no) left++;
+        if (size[k] > 4 * no + 4) more++;
+      }
+      if (left <= 4 && more == 0) {
+        quad = left > 0;
+        break;
+      }
+    }
+    int nq = 0;
+    for (int k = 0; k < 8 && nq < 4; k++)
+      if (size[k] > 4 * no) qc[nq++] = k;
+    for (int k = 7; k >= 0 && nq < 4; k--)
+      if (size[k] <= 4 * no) qc[nq++] = k;
+  }
+};
+template <int P>
+struct OConst {
+  static constexpr OLayout<P> O{};
+  static constexpr int NO = O.no, QUAD = O.quad, NSTEP = NO + QUAD;
+  static constexpr int BS = NO * 32 + QUAD * 16;       // floats of a stored box
+  // 16-byte fragments of an operator: an octet's hi and lo apart, a quad's in one
+  static constexpr int FRS = 8 * 2 * 64, FRQ = 8 * 64, FRO = NO * FRS + QUAD * FRQ;
+  static constexpr int ROWS = 8 * OLayout<P>::RW;      // partial sums per target
+};
+// largest |multipole| after scaling: sums of 4 stay below 2^15 in FP16
+constexpr int ORB_TOP = 13;
+// base offset of product o for a target of parity class cls (bits x, y, z) and
+// the operator's index in [0, NORBOP)
+void orbit_offset(int o, int cls, int* d);
+int orbit_op_index(const int* d);
+bool m2l_orbit_supported(int p);
+// operator fragments of the orbit kernel from all 316 k-major FP64 operators,
+// scaled by 2^sa_e: per operator [octet][row class][hi, lo][lane], then the quad
+// step's [row class][lane] with hi and lo in one fragment
+void orbit_fragments(const double* kmaj, int p, int sa_e, std::vector<uint4>& out);
+size_t orbit_frag_count(int p);
+
 // One M2L launch can cover several levels: workgroups [wg0, wg0 + nwg) of
 // the grid run level `lev` with that level's tiles, splits and buffers.
 // FP16 form: Mh (split multipoles), opH (split operators, fragment order),
@@ -133,7 +219,7 @@ struct MSplitLevels {
   unsigned* mmax[MAXL + 1];
   long off[MAXL + 2];
   int nl;
-  int wide;  // layout of the 32x32x16 kernel (WLayout), else HLayout
+  int wide;  // 1: layout of the 32x32x16 kernel (WLayout), 2: orbit kernel (OLayout, FP32), else HLayout
 };
 
 // m2l_split.hip
@@ -148,7 +234,14 @@ bool split_db_fits(int p);
 // (64 targets per wave), 4 waves and two buffers; p with split_wide_fits
 int launch_m2l_wide(int p, const M2LLaunch& A, int nwg, int wpg, int nt, hipStream_t stream);
 bool split_wide_fits(int p);
+// the orbit form: workgroups of ORB_WPG waves of 16 targets; partial sums per split
+// and target in row-class order (launch_orbit_reduce puts them into the locals)
+int launch_morder(int p, const MSplitLevels& S, hipStream_t stream);
+int launch_m2l_orbit(int p, const M2LLaunch& A, int nwg, const int4* orbtab, hipStream_t stream);
+int launch_orbit_reduce(int p, const M2LLaunch& A, hipStream_t stream);
 void split_fragments_wide(const double* kmaj, int count, int p, int sa_e, std::vector<uint4>& out);
+// floats of one stored box of the orbit kernel (0: not built for p)
+size_t orbit_box_floats(int p);
 // 16-byte fragments of one split operator; halfs of one split box
 inline size_t split_frag_count(int p) {
   const int P2 = p * p, MT = (P2 + 15) / 16, KS = (P2 + 3) / 4, SEG = KS + (KS & 1), KH = (3 * SEG + 7) / 8;
@@ -157,7 +250,8 @@ inline size_t split_frag_count(int p) {
 inline size_t split_box_halfs(int p) {
   const int KS = (p * p + 3) / 4, SEG = KS + (KS & 1);
   const int KS2 = (p * p + 1) / 2, SEG2 = KS2 + (KS2 & 1);
-  return std::max<size_t>((size_t)4 * ((2 * SEG + 7) / 8 * 8), (size_t)2 * ((2 * SEG2 + 7) / 8 * 8));
+  const size_t h = std::max<size_t>((size_t)4 * ((2 * SEG + 7) / 8 * 8), (size_t)2 * ((2 * SEG2 + 7) / 8 * 8));
+  return std::max(h, orbit_box_floats(p) * 2);
 }
 // operator fragments of the split form from k-major FP64 operators (count
 // of them, P2 x P2 each, element (row i, column k) at [k P2 + i]), scaled by

@@ -686,16 +686,18 @@ Engine::M2LVariant Engine::m2l_variant(int lev) const {
   if (v.nt <= 0) v.nt = 1;
   // default: the FP16 split kernel where it applies (FP32 Laplace engine,
   // EXACT, p 6..12), else LDS staging
-  if (v.pa < 0) v.pa = (split_ok && !yk && !hh && !fp64) ? (wide_ok ? 5 : 4) : 0;
+  if (v.pa < 0) v.pa = (split_ok && !yk && !hh && !fp64) ? (orb_ok && orbit_fits() ? 6 : wide_ok ? 5 : 4) : 0;
   if (v.wpg <= 0) v.wpg = 8;
   if (const char* e = getenv("FMMX_M2L_NT")) v.nt = atoi(e) == 4 ? 4 : atoi(e) == 2 ? 2 : 1;
-  if (const char* e = getenv("FMMX_M2L_PA")) v.pa = std::max(0, std::min(5, atoi(e)));
+  if (const char* e = getenv("FMMX_M2L_PA")) v.pa = std::max(0, std::min(6, atoi(e)));
   if (const char* e = getenv("FMMX_M2L_WPG")) v.wpg = atoi(e) == 4 ? 4 : atoi(e) == 16 ? 16 : 8;
   if (v.pa >= 3) {
     // FP16 split kernel: Laplace FP32 engine, p 6..12; two operator buffers
     // with one N-tile and 8 waves where they fit LDS
     if (!split_ok || yk || hh || fp64) v.pa = 0;
+    else if (v.pa == 6 && !(orb_ok && orbit_fits())) v.pa = wide_ok ? 5 : 4;
     else if (v.pa == 5 && !wide_ok) v.pa = 4;
+    if (v.pa == 6) v.nt = 1, v.wpg = ORB_WPG;
     if (v.pa == 4 && !split_db_fits(p)) v.pa = 3;
     // 32 targets per wave: 8 waves (two buffers) or 4 (one); 64 targets per
     // wave (nt 4): 4 waves, two buffers
@@ -731,6 +733,12 @@ Engine::M2LVariant Engine::m2l_variant(int lev) const {
       for (int c = 0; c < 8; c++) cmax = std::max(cmax, cls_cnt_h[lev][c]);
       const int tpc = std::max(1, (cmax + 16 * v.wpg * v.nt - 1) / (16 * v.wpg * v.nt));
       v.nsplit = 1024 / (8 * tpc);
+      // the orbit kernel: 63 products, and each workgroup starts with a copy
+      // of most of an operator; levels of a few tiles gain from more than 8
+      // splits (latency), larger ones lose (N = 1M, level 4 of 5: 8 splits
+      // 0.331 ms for the launch, 16 splits 0.341; a sphere's leaf level of
+      // 4,639 boxes 0.104 against 0.125)
+      if (v.pa == 6 && tpc > 1) v.nsplit = std::min(v.nsplit, 8);
     }
   }
   v.nsplit = std::max(1, std::min(16, v.nsplit));
@@ -810,15 +818,18 @@ void launch_m2l(const M2LLaunch& A, int nwg, int nt, int pa, int wpg, hipStream_
 // launch shape with each level's offset splits: levels with splits write
 // partial sums (reduced afterwards in fixed order), the others write their
 // locals; the L2L chain then adds the parents' locals level by level.
+// the orbit kernel addresses a level's stored boxes with 32-bit byte offsets
+bool Engine::orbit_fits() const { return ((size_t)sj.nb[lmax] + 1) * orbit_box_floats(p) * 4 < ((size_t)1 << 32); }
+
 bool Engine::m2l_split(int lev) const { return !fp64 && !hh && !yk && m2l_variant(lev).pa >= 3; }
 
 // The FP16 split kernel's inputs for levels [l0, l1]: the multipoles of every
 // level split into hi/lo pairs scaled by 2^(14 - exponent of the level's
 // largest magnitude), one pair of launches for all levels
-int Engine::run_msplit(int l0, int l1, bool wide) {
+int Engine::run_msplit(int l0, int l1, int form) {
   MSplitLevels S{};
   S.off[0] = 0;
-  S.wide = wide ? 1 : 0;
+  S.wide = form == 6 ? 2 : form == 5 ? 1 : 0;
   int rc = mmax_buf.ensure((MAXL + 1) * 4);
   if (rc) return rc;
   for (int lev = l0; lev <= l1; lev++) {
@@ -841,14 +852,17 @@ int Engine::run_msplit(int l0, int l1, bool wide) {
 // split shape (staging 3, 4) the multipoles are split first.
 int Engine::run_m2l_all(int l0) {
   const M2LVariant leaf = m2l_variant(lmax);
-  const bool split = leaf.pa >= 3;
+  const bool split = leaf.pa >= 3, orbit = leaf.pa == 6;
+  // floats of a target's partial sums (the orbit form always goes through them)
+  const size_t rows = orbit ? 8 * OLayout<2>::RW : P2;
   M2LLaunch A{};
   size_t need = 0;
   for (int lev = l0; lev <= lmax; lev++)
-    if (si.nb[lev] > 0 && sj.nb[lev] > 0 && m2l_splits(lev) > 1) need += (size_t)m2l_splits(lev) * si.nb[lev] * P2;
+    if (si.nb[lev] > 0 && sj.nb[lev] > 0 && (orbit || m2l_splits(lev) > 1))
+      need += (size_t)m2l_splits(lev) * si.nb[lev] * rows;
   int rc = m2l_part.ensure(std::max<size_t>(need, 1) * 4);
   if (rc) return rc;
-  if (split && (rc = run_msplit(l0, lmax, leaf.pa == 5))) return rc;
+  if (split && ((rc = upload_split(leaf.pa)) || (rc = run_msplit(l0, lmax, leaf.pa)))) return rc;
   size_t off = 0;
   int wg = 0;
   for (int lev = l0; lev <= lmax; lev++) {
@@ -860,7 +874,8 @@ int Engine::run_m2l_all(int l0) {
       continue;
     }
     const int ns = m2l_splits(lev);
-    A.lv[A.nlv] = m2l_desc(lev, leaf.nt, leaf.wpg, ns, ns > 1 ? m2l_part.as<float>() + off : nullptr, 1, wg);
+    A.lv[A.nlv] = m2l_desc(lev, leaf.nt, leaf.wpg, ns, orbit || ns > 1 ? m2l_part.as<float>() + off : nullptr, 1, wg);
+    if (orbit) A.lv[A.nlv].opH = op_m2l_o.as<uint4>();
     if (leaf.pa == 4) A.lv[A.nlv].offtab = offtab_s.as<int4>();
     if (leaf.pa == 5) {
       A.lv[A.nlv].offtab = offtab.as<int4>();
@@ -868,15 +883,16 @@ int Engine::run_m2l_all(int l0) {
     }
     wg += A.lv[A.nlv].nwg;
     A.nlv++;
-    if (ns > 1) off += (size_t)ns * nl;
+    if (orbit || ns > 1) off += (size_t)ns * nb * rows;
   }
   if (A.nlv == 0) return FMMX_OK;
   return dispatch_p(p, [&](auto pc) -> int {
     constexpr int P = decltype(pc)::value;
     if (per_phase) FMMX_HIP(hipEventRecord(ev[8], stream));
     if (split) {
-      int r2 = leaf.pa == 5 ? launch_m2l_wide(p, A, wg, leaf.wpg, leaf.nt, stream)
-                            : launch_m2l_split(p, A, wg, leaf.nt, leaf.wpg, leaf.pa == 4, stream);
+      int r2 = orbit          ? launch_m2l_orbit(p, A, wg, orbtab.as<int4>(), stream)
+               : leaf.pa == 5 ? launch_m2l_wide(p, A, wg, leaf.wpg, leaf.nt, stream)
+                              : launch_m2l_split(p, A, wg, leaf.nt, leaf.wpg, leaf.pa == 4, stream);
       if (r2) return r2;
     } else {
       launch_m2l<P>(A, wg, leaf.nt, leaf.pa, leaf.wpg, stream);
@@ -885,6 +901,7 @@ int Engine::run_m2l_all(int l0) {
       FMMX_HIP(hipEventRecord(ev[9], stream));
       m2l_timed = true;
     }
+    if (orbit) return launch_orbit_reduce(p, A, stream);
     // the partial sums of every level with splits, one launch
     ReduceLevels R{};
     R.off[0] = 0;
@@ -936,11 +953,13 @@ int Engine::run_m2l(int lev, bool init, int phase) {
     return FMMX_OK;
   }
   if (phase == 1 && nsplit < 2) return fail(FMMX_ESTATE, "M2L partial sums need offset splits");
-  if (nsplit > 1) {
-    int rc = part_buf->ensure((size_t)nsplit * nl * es);
+  const bool orbit = !fp64 && !hh && m2l_variant(lev).pa == 6;
+  if (orbit && phase == 1) return fail(FMMX_ESTATE, "the orbit M2L reduces with its launch");
+  if (nsplit > 1 || orbit) {
+    int rc = part_buf->ensure(orbit ? (size_t)nsplit * nb * 8 * OLayout<2>::RW * es : (size_t)nsplit * nl * es);
     if (rc) return rc;
   }
-  int rc2 = FMMX_OK;
+
   const int gsh = group_shift(lev);
   if (hh) {
     // split complex expansions: D = 2 p^2, k-major operators per level, on the
@@ -997,6 +1016,10 @@ int Engine::run_m2l(int lev, bool init, int phase) {
                                                                           lexp[lev].as<double>(), init ? 1 : 0);
     } else if constexpr (P <= P_ALL) {
       const M2LVariant var = m2l_variant(lev);
+      if (var.pa >= 3) {
+        int r2 = upload_split(var.pa);
+        if (r2) return r2;
+      }
       M2LLaunch A{};
       A.nlv = 1;
       A.lv[0] = m2l_desc(lev, var.nt, var.wpg, nsplit, part_buf->as<float>(), init ? 1 : 0, 0);
@@ -1005,15 +1028,17 @@ int Engine::run_m2l(int lev, bool init, int phase) {
         A.lv[0].offtab = offtab.as<int4>();
         A.lv[0].opH = op_m2l_w.as<uint4>();
       }
+      if (orbit) A.lv[0].opH = op_m2l_o.as<uint4>();
       if (var.pa >= 3) {
-        int r2 = run_msplit(lev, lev, var.pa == 5);
+        int r2 = run_msplit(lev, lev, var.pa);
         if (r2) return r2;
       }
       const bool tmark = per_phase && lev == lmax;
       if (tmark) FMMX_HIP(hipEventRecord(ev[8], stream));
       if (var.pa >= 3) {
-        int r2 = var.pa == 5 ? launch_m2l_wide(p, A, A.lv[0].nwg, var.wpg, var.nt, stream)
-                             : launch_m2l_split(p, A, A.lv[0].nwg, var.nt, var.wpg, var.pa == 4, stream);
+        int r2 = orbit         ? launch_m2l_orbit(p, A, A.lv[0].nwg, orbtab.as<int4>(), stream)
+                 : var.pa == 5 ? launch_m2l_wide(p, A, A.lv[0].nwg, var.wpg, var.nt, stream)
+                               : launch_m2l_split(p, A, A.lv[0].nwg, var.nt, var.wpg, var.pa == 4, stream);
         if (r2) return r2;
       } else {
         launch_m2l<P>(A, A.lv[0].nwg, var.nt, var.pa, var.wpg, stream);
@@ -1022,9 +1047,13 @@ int Engine::run_m2l(int lev, bool init, int phase) {
         FMMX_HIP(hipEventRecord(ev[9], stream));
         m2l_timed = true;
       }
-      if (nsplit > 1 && phase == 0)
+      if (orbit) {
+        int r2 = launch_orbit_reduce(p, A, stream);
+        if (r2) return r2;
+      } else if (nsplit > 1 && phase == 0) {
         k_m2l_reduce<float><<<(int)((nl + 255) / 256), 256, 0, stream>>>(nl, nsplit, part_buf->as<float>(),
                                                                          lexp[lev].as<float>(), init ? 1 : 0);
+      }
     }
     FMMX_HIP(hipGetLastError());
     return FMMX_OK;

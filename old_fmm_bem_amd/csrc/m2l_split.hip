@@ -879,7 +879,10 @@ int launch_msplit(int p, const MSplitLevels& S, hipStream_t stream) {
     k_msplit_max<P><<<nblk, MS_T, 0, stream>>>(S);
     if (S.off[S.nl] * 4 * (HLayout<P>::GH / 2) >= (1L << 32))
       return fail(FMMX_EUNSUPPORTED, "too many boxes for the multipole split");
-    if (S.wide) {
+    if (S.wide == 2) {
+      int rc = launch_morder(p, S, stream);
+      if (rc) return rc;
+    } else if (S.wide) {
       const long nw = S.off[S.nl] * 2 * (WLayout<P>::GH / 2);
       k_msplit<P, WLayout<P>, 2><<<(int)((nw + MS_T - 1) / MS_T), MS_T, 0, stream>>>(S);
     } else {

@@ -2,7 +2,10 @@
 // (m2l_split.hip): the operators' FP16 hi/lo split in the kernels' fragment
 // orders and the power-of-two scale that keeps them in range.  Plain host
 // C++ (no device code), so that it also builds under the sanitizers.
+#include <algorithm>
+#include <array>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 #include "m2l.h"
@@ -109,6 +112,108 @@ void split_fragments_wide(const double* kmaj, int count, int p, int sa_e, std::v
                          h[6] | (uint32_t)h[7] << 16);
         }
   }
+}
+
+// ---- reflection orbits ------------------------------------------------
+bool m2l_orbit_supported(int p) { return p >= 6 && p <= 10; }
+
+namespace {
+template <class F>
+auto with_orbit_p(int p, F&& f) {
+  switch (p) {
+    case 6: return f(OConst<6>{}, std::integral_constant<int, 6>{});
+    case 7: return f(OConst<7>{}, std::integral_constant<int, 7>{});
+    case 8: return f(OConst<8>{}, std::integral_constant<int, 8>{});
+    case 9: return f(OConst<9>{}, std::integral_constant<int, 9>{});
+    default: return f(OConst<10>{}, std::integral_constant<int, 10>{});
+  }
+}
+}  // namespace
+
+void orbit_offset(int o, int cls, int* d) {
+  // axis a in D: component 1 or 2 (both signs), else 0 or +-3 (the sign a
+  // target of this parity sees); bit a of the choice picks the larger, and the
+  // choice 0 (every |component| at most 1) is the near field
+  const int D = orb_mask(o), k = o - orb_start(D), half = k / 7, pick = k % 7 + 1;
+  const int axes = half > 0 ? 7 : D;  // the halves: z doubled too, one sign each
+  for (int a = 0; a < 3; a++) {
+    const int big = (pick >> a) & 1;
+    if ((axes >> a) & 1) d[a] = 1 + big;
+    else d[a] = !big ? 0 : (cls >> a) & 1 ? 3 : -3;
+  }
+  if (half == 2) d[2] = -d[2];
+}
+
+namespace {
+// the distinct base offsets over all classes, in order of first appearance
+const std::vector<std::array<int, 3>>& orbit_ops() {
+  static const std::vector<std::array<int, 3>> v = [] {
+    std::vector<std::array<int, 3>> u;
+    for (int cls = 0; cls < 8; cls++)
+      for (int o = 0; o < NORB; o++) {
+        std::array<int, 3> d;
+        orbit_offset(o, cls, d.data());
+        if (std::find(u.begin(), u.end(), d) == u.end()) u.push_back(d);
+      }
+    return u;
+  }();
+  return v;
+}
+}  // namespace
+
+int orbit_op_index(const int* d) {
+  const auto& u = orbit_ops();
+  const auto it = std::find(u.begin(), u.end(), std::array<int, 3>{d[0], d[1], d[2]});
+  return it == u.end() ? -1 : (int)(it - u.begin());
+}
+
+size_t orbit_frag_count(int p) {
+  return with_orbit_p(p, [](auto oc, auto) -> size_t { return decltype(oc)::FRO; });
+}
+
+size_t orbit_box_floats(int p) {
+  if (!m2l_orbit_supported(p)) return 0;
+  return with_orbit_p(p, [](auto oc, auto) -> size_t { return decltype(oc)::BS; });
+}
+
+void orbit_fragments(const double* kmaj, int p, int sa_e, std::vector<uint4>& out) {
+  with_orbit_p(p, [&](auto oc, auto pc) -> int {
+    using OC = decltype(oc);
+    constexpr int P2 = decltype(pc)::value * decltype(pc)::value;
+    const auto& O = OC::O;
+    out.assign((size_t)NORBOP * OC::FRO, make_uint4(0u, 0u, 0u, 0u));
+    const auto& ops = orbit_ops();
+    for (size_t oi = 0; oi < ops.size(); oi++) {
+      const double* A = kmaj + (size_t)offset_index(ops[oi][0], ops[oi][1], ops[oi][2]) * P2 * P2;  // (i, k) at [k P2 + i]
+      uint4* dst = &out[oi * OC::FRO];
+      for (int s = 0; s < OC::NSTEP; s++)
+        for (int c = 0; c < 8; c++)
+          for (int l = 0; l < 64; l++) {
+            const int i = O.slot[c][l & 15], g = l >> 4;
+            uint16_t h[2][8] = {};
+            for (int t = 0; t < 8; t++) {
+              const bool q = s == OC::NO;  // the quad step: hi words, lo words
+              const int kc = q ? O.qc[t & 3] : t, mem = 4 * s + g;
+              const int k = mem < O.size[kc] ? O.slot[kc][mem] : -1;
+              if (i < 0 || k < 0) continue;
+              const double a = std::ldexp(A[(size_t)k * P2 + i], sa_e);
+              const uint16_t hi = to_half(a), lo = to_half(a - from_half(hi));
+              h[0][t] = q && t >= 4 ? lo : hi;
+              h[1][t] = lo;
+            }
+            auto frag = [&](int e) {
+              return make_uint4(h[e][0] | (uint32_t)h[e][1] << 16, h[e][2] | (uint32_t)h[e][3] << 16,
+                                h[e][4] | (uint32_t)h[e][5] << 16, h[e][6] | (uint32_t)h[e][7] << 16);
+            };
+            if (s < OC::NO) {
+              for (int e = 0; e < 2; e++) dst[s * OC::FRS + (c * 2 + e) * 64 + l] = frag(e);
+            } else {
+              dst[OC::NO * OC::FRS + c * 64 + l] = frag(0);
+            }
+          }
+    }
+    return 0;
+  });
 }
 
 }  // namespace fmmx
