@@ -403,7 +403,10 @@ std::shared_ptr<OpSet> get_hh_ops(int p, double k, float rd, int lmax) {
   S->l2l.assign((size_t)nt_lev * 8 * dq, 0.0);
   S->nlev = lmax - 1;
   S->m2l_kmaj.resize((size_t)S->nlev * NOFF * dq);
-  // FP32 engine: MFMA fragment order of the D x D operators
+  // FP32 engine: P2 x P2 translations and the D x D M2L in MFMA fragment order
+  const size_t sq = (size_t)P2 * P2, fr = (size_t)((P2 + 3) / 4) * ((P2 + 15) / 16) * 64;
+  S->m2m_frag.assign((size_t)nt_lev * 8 * fr, 0.0);
+  S->l2l_frag.assign((size_t)nt_lev * 8 * fr, 0.0);
   const size_t frh = (size_t)(D / 4) * ((D + 15) / 16) * 64;
   S->m2l_frag.resize((size_t)S->nlev * NOFF * frh);
   const int ntr = lmax > 2 ? (lmax - 2) * 8 : 0, njobs = ntr + S->nlev * NOFF;
@@ -420,6 +423,13 @@ std::shared_ptr<OpSet> get_hh_ops(int p, double k, float rd, int lmax) {
           for (int r = 0; r < D; r++)
             for (int c = 0; c < D; c++) M[(size_t)pos(c) * VH + pos(r)] = A[(size_t)r * D + c];
           transpose_into(B.data(), D, &S->l2l[((size_t)li * 8 + o) * dq]);
+          // regular re-expansions act alike on both parts and do not mix them:
+          // the upper left block in fragment order serves the FP32 engine
+          std::vector<double> U(sq);
+          for (const auto& [op, dst] : {std::pair(&A, &S->m2m_frag), std::pair(&B, &S->l2l_frag)}) {
+            for (int r = 0; r < P2; r++) std::copy(&(*op)[(size_t)r * D], &(*op)[(size_t)r * D] + P2, &U[(size_t)r * P2]);
+            fragment_into(U.data(), P2, &(*dst)[((size_t)li * 8 + o) * fr]);
+          }
         } else {
           const int jj = j - ntr, li = jj / NOFF, oi = jj % NOFF;
           int d[3];
@@ -661,7 +671,7 @@ int Engine::upload_helmholtz_operators() {
         (rc = upload<double>(hop_m2l, S->m2l_kmaj, stream)))
       return rc;
   } else {
-    if ((rc = upload<float>(hop_m2m, S->m2m, stream)) || (rc = upload<float>(hop_l2l, S->l2l, stream)) ||
+    if ((rc = upload<float>(hop_m2m, S->m2m_frag, stream)) || (rc = upload<float>(hop_l2l, S->l2l_frag, stream)) ||
         (rc = upload<float>(hop_m2l, S->m2l_frag, stream)))
       return rc;
   }

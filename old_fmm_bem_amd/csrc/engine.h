@@ -159,8 +159,9 @@ struct Engine {
   // Helmholtz (FMMX_HELMHOLTZ): wavenumber, imaginary charges (key order) and
   // the operator sets per level on split expansions (two parts: the fields
   // of the real and of the imaginary charges, locals of Re and Im of the
-  // potential): M2M (2 VS)^2 by parent level 2..lmax-1, L2L (2 P2)^2 by child
-  // level 3..lmax, M2L (2 P2)^2 k-major by level
+  // potential): FP64 M2M (2 VS)^2 by parent level 2..lmax-1, L2L (2 P2)^2 by
+  // child level 3..lmax, M2L (2 P2)^2 k-major by level; FP32 M2M and L2L P2^2 in
+  // MFMA fragment order (one real operator for both parts)
   double hk = 0;
   bool hh = false;  // the evaluation in progress is Helmholtz
   DevBuf qs2, hop_m2m, hop_l2l, hop_m2l;
@@ -283,13 +284,15 @@ struct Engine {
   size_t frag_size() const { return (size_t)((P2 + 3) / 4) * ((P2 + 15) / 16) * 64; }
   template <class T>
   const T* m2m_ops(int parent_lev) const {
-    if (hh) return hop_m2m.as<T>() + (size_t)(parent_lev - 2) * 8 * 4 * VS * VS;
+    if (hh && fp64) return hop_m2m.as<T>() + (size_t)(parent_lev - 2) * 8 * 4 * VS * VS;
+    if (hh) return hop_m2m.as<T>() + (size_t)(parent_lev - 2) * 8 * frag_size();
     const size_t per = fp64 ? (size_t)VS * VS : frag_size();
     return yk ? yop_m2m.as<T>() + (size_t)(parent_lev - 2) * 8 * per : op_m2m.as<T>();
   }
   template <class T>
   const T* l2l_ops(int child_lev) const {
-    if (hh) return hop_l2l.as<T>() + (size_t)(child_lev - 3) * 8 * 4 * P2 * P2;
+    if (hh && fp64) return hop_l2l.as<T>() + (size_t)(child_lev - 3) * 8 * 4 * P2 * P2;
+    if (hh) return hop_l2l.as<T>() + (size_t)(child_lev - 3) * 8 * frag_size();
     const size_t per = fp64 ? (size_t)P2 * P2 : frag_size();
     return yk ? yop_l2l.as<T>() + (size_t)(child_lev - 3) * 8 * per : op_l2l.as<T>();
   }
