@@ -35,11 +35,13 @@ struct CountSrc {
   const int* cnt[2];  // box counts of both sides
   const int* cls;     // target boxes per level and class
   const int* bad;     // coordinates outside the root cube
+  int* p2p;           // counter of the P2P work items, cleared
 };
 constexpr int RB_CLS = 2 * (MAXL + 1) + 1;
 static_assert(RB_CLS + 8 * (MAXL + 1) <= RB_INTS, "readback buffer");
 __global__ void k_pack_counts(CountSrc src, int lmax, int* __restrict__ out) {
   const int t = threadIdx.x;
+  if (t == 0) *src.p2p = 0;
   if (t < 2 * (MAXL + 1)) {
     const int* c = src.cnt[t / (MAXL + 1)];
     out[t] = c ? c[t % (MAXL + 1)] : 0;
@@ -849,9 +851,14 @@ int Engine::set_points(int ni, const float* xi, const float* yi, const float* zi
   cs.cnt[1] = nj > 0 ? sj.cnt.as<int>() : nullptr;
   cs.cls = ni > 0 ? si.clscnt.as<int>() : nullptr;
   cs.bad = bad_flag.as<int>();
+  if ((rc = p2p_count.ensure(4))) return rc;
+  cs.p2p = p2p_count.as<int>();
   k_pack_counts<<<1, 64, 0, stream>>>(cs, lmax, rb_dev.as<int>());
   FMMX_HIP(hipMemcpyAsync(rb_host, rb_dev.p, RB_INTS * 4, hipMemcpyDeviceToHost, stream));
-  FMMX_HIP(hipStreamSynchronize(stream));
+  // the near field's work items run while the host takes up the counts
+  FMMX_HIP(hipEventRecord(ev[14], stream));
+  if ((rc = build_p2p_items())) return rc;
+  FMMX_HIP(hipEventSynchronize(ev[14]));
   if (rb_host[2 * (MAXL + 1)]) return fail(FMMX_EINVAL, "coordinates outside the root cube or not finite");
   for (int l = 2; l <= lmax; l++) {
     si.nb[l] = rb_host[l];

@@ -209,6 +209,12 @@ struct Engine {
   fmmx_stats stats{};
   int64_t p2p_pairs = 0, m2l_pairs = 0;
 
+  // work items of P2P (leaf, first target) of the tree in use, and the bound
+  // (FMMX_P2P_SMALL or its default; whether set) they were built for
+  DevBuf p2p_items, p2p_count;
+  double p2p_bound[2] = {-1, 0};
+  int build_p2p_items();
+
   ~Engine();
   int init(const fmmx_config* c, int dev, void* stream);
   int set_points(int ni, const float* xi, const float* yi, const float* zi, const float* nxi, const float* nyi,

@@ -86,11 +86,73 @@ __device__ __forceinline__ void pair(float xi, float yi, float zi, float nxi, fl
 // TPT lanes per target (2: leaves of at most about 32 targets, one wave per
 // workgroup): the lanes of a target take alternating staged sources and add
 // their sums at the end, so a half-empty leaf does not idle half the wave.
-// With TPT 2 each pass over the leaf's targets picks its own lanes per target
-// (2, 4, 8 or 16) from the targets it has left, so a pass of a few targets
-// (a leaf of 33-40, or of 10) still keeps the wave's lanes busy.
+// With TPT 2 each item picks its own lanes per target (2, 4, 8 or 16) from the
+// targets it has, so an item of a few targets (a leaf of 10, the rest of one of
+// 33-40) still keeps the wave's lanes busy.
+//
+// A workgroup takes work items, each a leaf and up to `tmax` of its targets
+// (k_p2p_items), so that a leaf of many targets is spread over the chip: 60,000
+// points in 64 leaves (lmax 2, REF) 4.13 -> 0.71 ms against one workgroup per
+// leaf; a Plummer cloud of 120,000 targets whose core leaves hold over 100
+// (lmax 7) 0.31 -> 0.14 ms.  With 32 targets per item the sums are those of
+// one workgroup per leaf in 32-target passes, bit for bit.
+
+// Shape of the near field for n targets in nb leaves: the one-wave form (lanes
+// per target chosen per item) or `lanes` lanes, one per target, and targets per
+// item.  One wave for leaves of at most `small` targets on average (measured
+// 36-47% less P2P time than one lane per target in 64/128-lane blocks at 46-61
+// targets per leaf; 256-lane blocks win above 96: 2.95 against 3.55 ms at 244
+// per leaf), and for every leaf size while 256-target blocks would leave the
+// chip idle.  Its items hold 32 targets (two lanes each), fewer where that
+// leaves the 1,024 SIMDs fewer than two waves each (1,000 points in 64 leaves:
+// 4 per item), and a quarter of that in leaves of over `heavy` targets, so that
+// an item's work (targets x sources) stays within a few times the others'.
+struct P2PShape {
+  int one_wave, lanes, tmax, heavy;
+};
+__host__ __device__ inline P2PShape p2p_shape(int n, int nb, double small, bool fixed) {
+  const double mean = (double)n / (nb > 0 ? nb : 1);
+  P2PShape s{};
+  s.one_wave = mean <= small || (!fixed && n / 256 + nb / 2 < 1024);
+  s.lanes = s.one_wave ? 64 : mean > 96 ? 256 : mean > 40 ? 128 : 64;
+  s.tmax = s.one_wave ? 32 : s.lanes;
+  if (s.one_wave)
+    while (s.tmax > 4 && n / s.tmax + nb < 2048) s.tmax /= 2;
+  s.heavy = !s.one_wave || mean > 1e8 ? 1 << 30 : mean > 16 ? (int)(4 * mean) : 64;
+  return s;
+}
+__device__ __forceinline__ int p2p_targets(int n, const P2PShape& s) {
+  return n <= s.heavy ? s.tmax : s.tmax > 8 ? s.tmax / 4 : s.tmax;
+}
+// items of all leaves (their number is read on the device: the launch precedes
+// the host's readback of it)
+__global__ __launch_bounds__(256) void k_p2p_items(int n_, const int* __restrict__ nb_, double small, int fixed,
+                                                   const int* __restrict__ first, const int* __restrict__ last,
+                                                   int2* __restrict__ items, int* __restrict__ count) {
+  const int nbi = *nb_;
+  const P2PShape sh = p2p_shape(n_, nbi, small, fixed != 0);
+  const int b = blockIdx.x * 256 + threadIdx.x, lane = threadIdx.x & 63;
+  int i0 = 0, n = 0, t = 1, c = 0;
+  if (b < nbi) {
+    i0 = first[b];
+    n = last[b] - i0 + 1;
+    t = p2p_targets(n, sh);
+    c = (n + t - 1) / t;
+  }
+  int s = c;  // inclusive sums over the wave: one atomic per wave
+  for (int d = 1; d < 64; d <<= 1) {
+    const int u = __shfl_up(s, d);
+    if (lane >= d) s += u;
+  }
+  int base = 0;
+  if (lane == 63) base = atomicAdd(count, s);
+  base = __shfl(base, 63) + s - c;
+  for (int k = 0; k < c; k++) items[base + k] = make_int2(b, i0 + k * t);
+}
+
 template <typename T, int NEQ, int CONV, int BS, int TPT = 1>
-__global__ __launch_bounds__(BS) void k_p2p(int nbi, const uint32_t* __restrict__ ikey, const uint32_t* __restrict__ jkey,
+__global__ __launch_bounds__(BS) void k_p2p(const int2* __restrict__ items, const int* __restrict__ nitems, P2PShape shape,
+                                            const uint32_t* __restrict__ ikey, const uint32_t* __restrict__ jkey,
                                             const int* __restrict__ ifirst, const int* __restrict__ ilast,
                                             const int* __restrict__ nij, const int* __restrict__ neij,
                                             const int* __restrict__ jfirst, const int* __restrict__ jlast,
@@ -115,18 +177,18 @@ __global__ __launch_bounds__(BS) void k_p2p(int nbi, const uint32_t* __restrict_
   __shared__ float4 sp[SB];
   __shared__ float4 sn[SN ? SB : 1];
   static_assert(TPT == 1 || (TPT == 2 && BS == 64), "two lanes per target within one wave");
-  const int b = blockIdx.x, tid = threadIdx.x;
-  if (b >= nbi) return;
-  const int i0 = ifirst[b], i1 = ilast[b], nn = nij[b];
-  for (int base = i0, tb = BS; base <= i1; base += tb) {
-    // lanes per target of this pass (uniform): TPT, or up to 16 (TPT 2) for
-    // the targets left
+  const int tid = threadIdx.x, ni = *nitems;
+  for (int it = blockIdx.x; it < ni; it += gridDim.x) {
+    const int2 item = items[it];
+    const int b = item.x, base = item.y, nn = nij[b];
+    const int i1 = min(ilast[b], base + p2p_targets(ilast[b] - ifirst[b] + 1, shape) - 1);
+    // lanes per target (uniform): TPT, or up to 16 (TPT 2) for few targets
     int tpt = TPT;
     if (TPT == 2) {
       const int m = i1 - base + 1;
       tpt = m > 16 ? 2 : m > 8 ? 4 : m > 4 ? 8 : 16;
     }
-    tb = BS / tpt;  // targets of this pass
+    const int tb = BS / tpt;  // targets the lanes cover
     const int tt = tid % tb, part = tid / tb;
     const int i = base + tt;
     const bool act = i <= i1;
@@ -330,38 +392,68 @@ __global__ void k_zero_d(long n, double* __restrict__ a) {
 
 }  // namespace
 
+namespace {
+__global__ void k_zero_i(int* a) {
+  if (threadIdx.x == 0) *a = 0;
+}
+constexpr double P2P_SMALL = 96.0;  // FMMX_P2P_SMALL sets the bound instead
+}  // namespace
+
+// The work items of the tree in use (p2p_count cleared before); box counts may
+// still be on the device only
+int Engine::build_p2p_items() {
+  const int n = si.n;
+  if (n == 0) return FMMX_OK;
+  const char* es = getenv("FMMX_P2P_SMALL");
+  p2p_bound[0] = es ? atof(es) : P2P_SMALL;
+  p2p_bound[1] = es ? 1.0 : 0.0;
+  const long nbmax = std::min<long>(n, 1L << (3 * lmax));
+  int rc = p2p_items.ensure(((size_t)nbmax + n / 4 + 1) * 8);
+  if (rc) return rc;
+  k_p2p_items<<<(int)((nbmax + 255) / 256), 256, 0, stream>>>(n, si.cnt.as<int>() + lmax, p2p_bound[0],
+                                                              p2p_bound[1] != 0, si.bfirst[lmax].as<int>(),
+                                                              si.blast.as<int>(), p2p_items.as<int2>(),
+                                                              p2p_count.as<int>());
+  FMMX_HIP(hipGetLastError());
+  return FMMX_OK;
+}
+
 int Engine::run_p2p(int neq) {
   const int nbi = si.nb[lmax];
   if (nbi == 0) return FMMX_OK;
   const double cc = neq == FMMX_YUKAWA ? c_yukawa() : c4();
   const bool ref = cfg.convention == FMMX_CONV_REF;
-  const double mean = (double)si.n / nbi;
   // Helmholtz: the imaginary charges ride in the source-normal slot, k in lambda's
   const float* nxj = neq == FMMX_HELMHOLTZ ? qs2.as<float>() : sj.nx.as<float>();
   const double kl = neq == FMMX_HELMHOLTZ ? hk : lam;
+  const char* es = getenv("FMMX_P2P_SMALL");
+  const P2PShape shape = p2p_shape(si.n, nbi, es ? atof(es) : P2P_SMALL, es != nullptr);
+  const double now[2] = {es ? atof(es) : P2P_SMALL, es ? 1.0 : 0.0};
+  int rc = FMMX_OK;
+  if (now[0] != p2p_bound[0] || now[1] != p2p_bound[1]) {
+    // the bound changed since the items were built
+    k_zero_i<<<1, 64, 0, stream>>>(p2p_count.as<int>());
+    if ((rc = build_p2p_items())) return rc;
+  }
+  // about the number of items (known on the device); each workgroup strides
+  const int grid = nbi + si.n / (2 * shape.tmax) + 1;
   auto go = [&](auto tag_t, auto neq_c, auto conv_c, auto bs_c, auto tpt_c) -> int {
     using T = typename decltype(tag_t)::type;
     constexpr int NEQ = decltype(neq_c)::value, CONV = decltype(conv_c)::value, BS = decltype(bs_c)::value;
     constexpr int TPT = decltype(tpt_c)::value;
-    k_p2p<T, NEQ, CONV, BS, TPT><<<nbi, BS, 0, stream>>>(
-        nbi, si.bkey[lmax].as<uint32_t>(), sj.bkey[lmax].as<uint32_t>(), si.bfirst[lmax].as<int>(), si.blast.as<int>(), nij.as<int>(), neij.as<int>(), sj.bfirst[lmax].as<int>(),
+    k_p2p<T, NEQ, CONV, BS, TPT><<<grid, BS, 0, stream>>>(
+        p2p_items.as<int2>(), p2p_count.as<int>(), shape, si.bkey[lmax].as<uint32_t>(), sj.bkey[lmax].as<uint32_t>(), si.bfirst[lmax].as<int>(), si.blast.as<int>(), nij.as<int>(), neij.as<int>(), sj.bfirst[lmax].as<int>(),
         sj.blast.as<int>(), si.x.as<float>(), si.y.as<float>(), si.z.as<float>(), si.nx.as<float>(), si.ny.as<float>(),
         si.nz.as<float>(), sj.x.as<float>(), sj.y.as<float>(), sj.z.as<float>(), qs.as<float>(), nxj,
         sj.ny.as<float>(), sj.nz.as<float>(), cc, vs.as<double>(), gxs.as<double>(), gys.as<double>(),
         gzs.as<double>(), kl);
     return FMMX_OK;
   };
-  // leaves of at most `small` targets on average: one wave per leaf with
-  // lanes per target chosen per pass (TPT 2; measured 36-47% less P2P time
-  // than one lane per target in 64/128-lane blocks at 46-61 targets per
-  // leaf); FMMX_P2P_SMALL sets the bound
-  double small = 96.0;
-  if (const char* e = getenv("FMMX_P2P_SMALL")) small = atof(e);
   auto by_bs = [&](auto t, auto nq, auto cv) -> int {
     using one = std::integral_constant<int, 1>;
-    if (mean <= small) return go(t, nq, cv, std::integral_constant<int, 64>{}, std::integral_constant<int, 2>{});
-    if (mean > 96) return go(t, nq, cv, std::integral_constant<int, 256>{}, one{});
-    if (mean > 40) return go(t, nq, cv, std::integral_constant<int, 128>{}, one{});
+    if (shape.one_wave) return go(t, nq, cv, std::integral_constant<int, 64>{}, std::integral_constant<int, 2>{});
+    if (shape.lanes == 256) return go(t, nq, cv, std::integral_constant<int, 256>{}, one{});
+    if (shape.lanes == 128) return go(t, nq, cv, std::integral_constant<int, 128>{}, one{});
     return go(t, nq, cv, std::integral_constant<int, 64>{}, one{});
   };
   auto by_conv = [&](auto t, auto nq) -> int {
@@ -375,7 +467,7 @@ int Engine::run_p2p(int neq) {
     if (neq == FMMX_GNI) return by_conv(t, std::integral_constant<int, FMMX_GNI>{});
     return by_conv(t, std::integral_constant<int, FMMX_GNJ>{});
   };
-  int rc = fp64 ? by_neq(tag<double>{}) : by_neq(tag<float>{});
+  rc = fp64 ? by_neq(tag<double>{}) : by_neq(tag<float>{});
   if (rc) return rc;
   FMMX_HIP(hipGetLastError());
   return FMMX_OK;
