@@ -145,7 +145,7 @@ __global__ __launch_bounds__(256) void k_p2p_items(int n_, const int* __restrict
     if (lane >= d) s += u;
   }
   int base = 0;
-  if (lane == 63) base = atomicAdd(count, s);
+  if (lane == 63 && s > 0) base = atomicAdd(count, s);
   base = __shfl(base, 63) + s - c;
   for (int k = 0; k < c; k++) items[base + k] = make_int2(b, i0 + k * t);
 }
