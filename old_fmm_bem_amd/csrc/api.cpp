@@ -198,6 +198,7 @@ struct OpSet {
   std::vector<uint4> m2l_wide;
   // the same split for the reflection-orbit kernel: its NORBOP operators
   std::vector<uint4> m2l_orbit;
+  std::vector<int> lev_e;  // scale exponents of per-level orbit operators
   int nlev = 1;
 };
 std::mutex g_cache_mu;
@@ -381,12 +382,14 @@ std::shared_ptr<OpSet> get_yuk_ops(int p, double lam, float rd, int lmax) {
 // Helmholtz operator sets keyed by (p, k, rd, lmax), on split expansions:
 // M2M per parent level 2..lmax-1 (padded multipole layout of both parts,
 // (2 VS)^2, k-major), L2L per child level 3..lmax ((2 P2)^2, k-major), M2L per
-// level 2..lmax (316 offsets, (2 P2)^2, k-major)
-std::map<std::tuple<int, double, float, int>, std::shared_ptr<OpSet>> g_hh_cache;
+// level 2..lmax (316 offsets, (2 P2)^2, k-major).  FP32: the real P2 x P2 block
+// of the translations in MFMA fragment order, and the blocks C and S of the M2L
+// operator [[C, -S], [S, C]] of the orbits' base offsets as FP16 hi/lo fragments
+std::map<std::tuple<int, double, float, int, bool>, std::shared_ptr<OpSet>> g_hh_cache;
 
-std::shared_ptr<OpSet> get_hh_ops(int p, double k, float rd, int lmax) {
+std::shared_ptr<OpSet> get_hh_ops(int p, double k, float rd, int lmax, bool fp64) {
   const int P2 = p * p, D = 2 * P2;
-  auto key = std::make_tuple(p, k, rd, lmax);
+  auto key = std::make_tuple(p, k, rd, lmax, fp64);
   {
     std::lock_guard<std::mutex> lk(g_cache_mu);
     auto it = g_hh_cache.find(key);
@@ -401,48 +404,72 @@ std::shared_ptr<OpSet> get_hh_ops(int p, double k, float rd, int lmax) {
     return t * VS + (r / KS) * KSP + r % KS;
   };
   const int nt_lev = std::max(1, lmax - 2);
-  S->m2m.assign((size_t)nt_lev * 8 * vq, 0.0);
-  S->l2l.assign((size_t)nt_lev * 8 * dq, 0.0);
   S->nlev = lmax - 1;
-  S->m2l_kmaj.resize((size_t)S->nlev * NOFF * dq);
-  // FP32 engine: P2 x P2 translations and the D x D M2L in MFMA fragment order
   const size_t sq = (size_t)P2 * P2, fr = (size_t)((P2 + 3) / 4) * ((P2 + 15) / 16) * 64;
-  S->m2m_frag.assign((size_t)nt_lev * 8 * fr, 0.0);
-  S->l2l_frag.assign((size_t)nt_lev * 8 * fr, 0.0);
-  const size_t frh = (size_t)(D / 4) * ((D + 15) / 16) * 64;
-  S->m2l_frag.resize((size_t)S->nlev * NOFF * frh);
-  const int ntr = lmax > 2 ? (lmax - 2) * 8 : 0, njobs = ntr + S->nlev * NOFF;
-  std::vector<std::thread> th;
-  unsigned nt = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
-  for (unsigned t = 0; t < nt; t++)
-    th.emplace_back([&, t] {
-      std::vector<double> A(dq), B(dq);
-      for (int j = (int)t; j < njobs; j += (int)nt) {
-        if (j < ntr) {
-          const int li = j / 8, o = j % 8, lc = 3 + li;
-          hh_op_m2m_l2l(p, k * (double)rd / (double)(1 << lc), o, A.data(), B.data());
+  const int noff = fp64 ? NOFF : NORBOP;
+  const size_t frg = orbit_gen_frags(p, 1);
+  std::vector<double> cs;  // FP32: C and S per (level, base offset)
+  if (fp64) {
+    S->m2m.assign((size_t)nt_lev * 8 * vq, 0.0);
+    S->l2l.assign((size_t)nt_lev * 8 * dq, 0.0);
+    S->m2l_kmaj.resize((size_t)S->nlev * NOFF * dq);
+  } else {
+    S->m2m_frag.assign((size_t)nt_lev * 8 * fr, 0.0);
+    S->l2l_frag.assign((size_t)nt_lev * 8 * fr, 0.0);
+    S->m2l_orbit.resize((size_t)S->nlev * NORBOP * frg);
+    cs.resize((size_t)S->nlev * NORBOP * 2 * sq);
+  }
+  const int ntr = lmax > 2 ? (lmax - 2) * 8 : 0, njobs = ntr + S->nlev * noff;
+  const unsigned nt = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
+  auto parallel = [&](auto&& f) {
+    std::vector<std::thread> th;
+    for (unsigned t = 0; t < nt; t++) th.emplace_back([&, t] { f((int)t); });
+    for (auto& x : th) x.join();
+  };
+  parallel([&](int t) {
+    std::vector<double> A(dq), B(dq), U(sq);
+    for (int j = t; j < njobs; j += (int)nt) {
+      if (j < ntr) {
+        const int li = j / 8, o = j % 8, lc = 3 + li;
+        hh_op_m2m_l2l(p, k * (double)rd / (double)(1 << lc), o, A.data(), B.data());
+        if (fp64) {
           double* M = &S->m2m[((size_t)li * 8 + o) * vq];
           for (int r = 0; r < D; r++)
             for (int c = 0; c < D; c++) M[(size_t)pos(c) * VH + pos(r)] = A[(size_t)r * D + c];
           transpose_into(B.data(), D, &S->l2l[((size_t)li * 8 + o) * dq]);
-          // regular re-expansions act alike on both parts and do not mix them:
-          // the upper left block in fragment order serves the FP32 engine
-          std::vector<double> U(sq);
-          for (const auto& [op, dst] : {std::pair(&A, &S->m2m_frag), std::pair(&B, &S->l2l_frag)}) {
-            for (int r = 0; r < P2; r++) std::copy(&(*op)[(size_t)r * D], &(*op)[(size_t)r * D] + P2, &U[(size_t)r * P2]);
-            fragment_into(U.data(), P2, &(*dst)[((size_t)li * 8 + o) * fr]);
-          }
-        } else {
-          const int jj = j - ntr, li = jj / NOFF, oi = jj % NOFF;
-          int d[3];
-          offset_vector(oi, d);
-          hh_op_m2l(p, k * (double)rd / (double)(1 << (li + 2)), d[0], d[1], d[2], A.data());
+          continue;
+        }
+        // regular re-expansions act alike on both parts and do not mix them
+        for (const auto& [op, dst] : {std::pair(&A, &S->m2m_frag), std::pair(&B, &S->l2l_frag)}) {
+          for (int r = 0; r < P2; r++) std::copy(&(*op)[(size_t)r * D], &(*op)[(size_t)r * D] + P2, &U[(size_t)r * P2]);
+          fragment_into(U.data(), P2, &(*dst)[((size_t)li * 8 + o) * fr]);
+        }
+      } else {
+        const int jj = j - ntr, li = jj / noff, oi = jj % noff;
+        int d[3];
+        if (fp64) offset_vector(oi, d);
+        else orbit_op_vector(oi, d);
+        hh_op_m2l(p, k * (double)rd / (double)(1 << (li + 2)), d[0], d[1], d[2], A.data());
+        if (fp64) {
           transpose_into(A.data(), D, &S->m2l_kmaj[((size_t)li * NOFF + oi) * dq]);
-          fragment_into(A.data(), D, &S->m2l_frag[((size_t)li * NOFF + oi) * frh]);
+        } else {
+          double* dst = &cs[((size_t)li * NORBOP + oi) * 2 * sq];
+          for (int r = 0; r < D; r++)
+            std::copy(&A[(size_t)r * D], &A[(size_t)r * D] + P2, dst + (size_t)r * P2);  // rows of C, then of S
         }
       }
+    }
+  });
+  if (!fp64) {
+    for (int li = 0; li < S->nlev; li++)
+      S->lev_e.push_back(split_scale_exp(&cs[(size_t)li * NORBOP * 2 * sq], (size_t)NORBOP * 2 * sq));
+    parallel([&](int t) {
+      for (int j = t; j < S->nlev * NORBOP; j += (int)nt) {
+        const double* C = &cs[(size_t)j * 2 * sq];
+        orbit_gen_fragments(C, C + sq, P2, p, S->lev_e[j / NORBOP], &S->m2l_orbit[(size_t)j * frg]);
+      }
     });
-  for (auto& x : th) x.join();
+  }
   std::lock_guard<std::mutex> lk(g_cache_mu);
   g_hh_cache[key] = S;
   return S;
@@ -666,7 +693,7 @@ int Engine::set_helmholtz(double k) {
 
 int Engine::upload_helmholtz_operators() {
   if (hops_lmax == lmax && hops_rd == rd && hops_k == hk) return FMMX_OK;
-  auto S = get_hh_ops(p, hk, rd, lmax);
+  auto S = get_hh_ops(p, hk, rd, lmax, fp64);
   int rc;
   if (fp64) {
     if ((rc = upload<double>(hop_m2m, S->m2m, stream)) || (rc = upload<double>(hop_l2l, S->l2l, stream)) ||
@@ -674,8 +701,11 @@ int Engine::upload_helmholtz_operators() {
       return rc;
   } else {
     if ((rc = upload<float>(hop_m2m, S->m2m_frag, stream)) || (rc = upload<float>(hop_l2l, S->l2l_frag, stream)) ||
-        (rc = upload<float>(hop_m2l, S->m2l_frag, stream)))
+        (rc = hop_m2l.ensure(S->m2l_orbit.size() * 16)))
       return rc;
+    FMMX_HIP(hipMemcpyAsync(hop_m2l.p, S->m2l_orbit.data(), S->m2l_orbit.size() * 16, hipMemcpyHostToDevice, stream));
+    FMMX_HIP(hipStreamSynchronize(stream));
+    for (int l = 2; l <= lmax; l++) hop_e[l] = S->lev_e[l - 2];
   }
   hops_lmax = lmax;
   hops_rd = rd;
@@ -933,6 +963,7 @@ int Engine::prepare(int neq) {
     if ((rc = mexp[l].ensure((size_t)std::max(1, sj.nb[l]) * VS * np * es)) ||
         (rc = lexp[l].ensure((size_t)std::max(1, si.nb[l]) * P2 * np * es)))
       return rc;
+    if (hh && !fp64 && (rc = mexp_h[l].ensure((size_t)(sj.nb[l] + 1) * orbit_gen_box_floats(p, 1) * 4))) return rc;
     if (split_ok && !hh && !fp64 && (rc = mexp_h[l].ensure((size_t)(sj.nb[l] + 1) * split_box_halfs(p) * 2)))
       return rc;
   }

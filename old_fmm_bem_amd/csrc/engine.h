@@ -161,7 +161,8 @@ struct Engine {
   // of the real and of the imaginary charges, locals of Re and Im of the
   // potential): FP64 M2M (2 VS)^2 by parent level 2..lmax-1, L2L (2 P2)^2 by
   // child level 3..lmax, M2L (2 P2)^2 k-major by level; FP32 M2M and L2L P2^2 in
-  // MFMA fragment order (one real operator for both parts)
+  // MFMA fragment order (one real operator for both parts), M2L the hi/lo
+  // fragments of the orbits' base operators by level
   double hk = 0;
   bool hh = false;  // the evaluation in progress is Helmholtz
   DevBuf qs2, hop_m2m, hop_l2l, hop_m2l;
@@ -215,6 +216,8 @@ struct Engine {
   double p2p_bound[2] = {-1, 0};
   int build_p2p_items();
 
+  int hop_e[MAXL + 1] = {};  // scale exponents of hop_m2l per level (FP32)
+
   ~Engine();
   int init(const fmmx_config* c, int dev, void* stream);
   int set_points(int ni, const float* xi, const float* yi, const float* zi, const float* nxi, const float* nyi,
@@ -263,12 +266,13 @@ struct Engine {
   M2LVariant m2l_variant(int lev) const;
   int m2l_splits(int lev) const { return m2l_variant(lev).nsplit; }
   int run_m2l(int lev, bool init, int phase = 0);
-  int run_m2l_all(int l0);  // FP32 MFMA: every level in one launch
+  int run_m2l_all(int l0);  // FP32: every level in one launch
+  int run_m2l_hh(int l0, int l1, bool init);  // FP32 Helmholtz, levels l0..l1 in one launch
   int run_msplit(int l0, int l1, int form);  // split multipoles for the FP16 kernels
   bool last_m2l_all = false;  // the last evaluation took that form
   bool m2l_timed = false;     // the last evaluation recorded ev[8], ev[9] around its M2L launch
   bool m2l_all_levels() const {
-    if (fp64 || hh) return false;
+    if (fp64) return false;
     const char* e = getenv("FMMX_M2L_FUSED");
     return !e || atoi(e) != 0;
   }

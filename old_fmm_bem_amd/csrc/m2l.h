@@ -99,6 +99,9 @@ struct WLayout {
 // largest magnitude of the scaled split operands (2^14)
 constexpr int SPLIT_TOP = 14;
 
+struct MSplitLevels;
+struct M2LLaunch;
+
 // Reflection orbits of the M2L offsets.  T_r (ReflMask) is diagonal, so the
 // real slots fall into 8 classes by their signs under the three reflections:
 // class kappa (bits x, y, z) holds the slots with T_r = (-1)^popcount(kappa & r).
@@ -172,6 +175,69 @@ struct OConst {
   static constexpr int FRS = 8 * 2 * 64, FRQ = 8 * 64, FRO = NO * FRS + QUAD * FRQ;
   static constexpr int ROWS = 8 * OLayout<P>::RW;      // partial sums per target
 };
+// The general form (m2l_orbit_gen.hip): row classes of more than 16 slots take
+// two 16-row tiles, and classes of more words than the octets hold put up to
+// two more words of each into one last octet (positions t, t + 4: words NO,
+// NO + 1 of class qc[t]).  HH: Helmholtz, split expansions of two parts, whose
+// operator is [[C, -S], [S, C]] for two real operators C and S.
+template <int P>
+struct GLayout {
+  OLayout<P> O;
+  int no, xtra;          // octets of every class, 1: a last octet of the larger ones
+  int qc[4];
+  int nt;                // row tiles
+  int tcls[16], trow[16];  // class and first row of a tile
+  constexpr GLayout() : O{}, no(0), xtra(0), qc{}, nt(0), tcls{}, trow{} {
+    for (no = 0;; no++) {
+      int left = 0, more = 0;
+      for (int k = 0; k < 8; k++) {
+        if (O.size[k] > 4 * no) left++;
+        if (O.size[k] > 4 * no + 8) more++;
+      }
+      if (left <= 4 && more == 0) {
+        xtra = left > 0;
+        break;
+      }
+    }
+    int nq = 0;
+    for (int k = 0; k < 8 && nq < 4; k++)
+      if (O.size[k] > 4 * no) qc[nq++] = k;
+    for (int k = 7; k >= 0 && nq < 4; k--)
+      if (O.size[k] <= 4 * no) qc[nq++] = k;
+    for (int k = 0; k < 8; k++)
+      for (int r = 0; r < O.size[k]; r += 16) {
+        tcls[nt] = k;
+        trow[nt++] = r;
+      }
+  }
+  // class and member of position t of lane group g at step s (member -1: none)
+  constexpr int cls(int s, int t) const { return s == no ? qc[t & 3] : t; }
+  constexpr int member(int s, int t, int g) const {
+    const int m = s == no ? 4 * (no + (t >> 2)) + g : 4 * s + g;
+    return m < O.size[cls(s, t)] ? m : -1;
+  }
+};
+template <int P, int HH>
+struct GConst {
+  static constexpr GLayout<P> L{};
+  static constexpr int P2 = P * P, PARTS = HH ? 2 : 1, NO = L.no, XTRA = L.xtra, NSTEP = NO + XTRA, NT = L.nt;
+  static constexpr int PBS = NSTEP * 32, BS = PARTS * PBS;  // floats of a stored part, box
+  static constexpr int CH = NT * PARTS * 2 * 64, FRO = NSTEP * CH;  // 16-byte fragments of a step, operator
+  static constexpr int ROWS = PARTS * NT * 16;                      // partial sums per target
+};
+// launchers of the general form; opset[lev]: fragments of that level's operators
+int launch_m2l_orbit_gen(int p, int hh, const M2LLaunch& A, int nwg, const int4* orbtab, hipStream_t stream);
+int launch_orbit_gen_order(int p, int hh, const MSplitLevels& S, hipStream_t stream);
+int launch_orbit_gen_reduce(int p, int hh, const M2LLaunch& A, hipStream_t stream);
+size_t orbit_gen_box_floats(int p, int hh);
+size_t orbit_gen_frags(int p, int hh);
+size_t orbit_gen_rows(int p, int hh);
+// fragments of one operator (C, and S for hh; row-major P2 x P2 blocks of leading
+// dimension ld), scaled by 2^sa_e
+void orbit_gen_fragments(const double* C, const double* S, int ld, int p, int sa_e, uint4* out);
+// the distinct base offsets of the orbits, NORBOP of them
+void orbit_op_vector(int i, int* d);
+
 // largest |multipole| after scaling: sums of 4 stay below 2^15 in FP16
 constexpr int ORB_TOP = 13;
 // base offset of product o for a target of parity class cls (bits x, y, z) and

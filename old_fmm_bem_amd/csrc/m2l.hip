@@ -351,169 +351,6 @@ __global__ __launch_bounds__(64 * WPG) void k_m2l(M2LLaunch A) {
   if (mypairs) atomicAdd(npairs, mypairs);
 }
 
-// Helmholtz M2L of the FP32 engine on MFMA (v_mfma_f32_16x16x4f32): split
-// complex expansions, D = 2 p^2 rows ([Re; Im] locals) and columns ([R; I]
-// multipoles), operators per level in fragment order.  The whole operator
-// (D^2 floats, 332 KB at p = 12) exceeds LDS, so it is staged in chunks of
-// HH_KC k-steps shared by the workgroup's waves; each wave keeps its 16
-// targets' source multipoles (D / 4 per lane) in registers and skips the
-// products of an offset for which none of its targets has a source box.  Tile,
-// class, split and XCD mapping as k_m2l.
-constexpr int HH_KC = 8;
-template <int P, int WPG>
-__global__ __launch_bounds__(64 * WPG) __attribute__((amdgpu_waves_per_eu(1, 2))) void k_m2l_hh(int lev, int nb, int nsplit, const int* __restrict__ cls_cnt,
-                                                     const uint32_t* __restrict__ ord,
-                                                     const uint32_t* __restrict__ ikey,
-                                                     const int* __restrict__ dense_j, const float* __restrict__ M,
-                                                     float* __restrict__ L, float* __restrict__ part,
-                                                     const float* __restrict__ opF, const int4* __restrict__ offtab,
-                                                     int init, int region, int gsh,
-                                                     unsigned long long* __restrict__ npairs) {
-  using ML = MLayout<P>;
-  constexpr int P2 = P * P, D = 2 * P2, MT = (D + 15) / 16, KS = D / 4, FR = KS * MT * 64;
-  constexpr int NCH = (KS + HH_KC - 1) / HH_KC, CHF = HH_KC * MT * 64;  // chunks, floats per chunk
-  constexpr int NTH = 64 * WPG, TN = 16 * WPG;
-  static_assert(P % 2 == 0 && KS * 2 == P2, "each lane's k-range lies in one part");
-  using V4 = f32x4;
-  // two chunk buffers: the next chunk is loaded into registers while the
-  // current one feeds the MFMAs, then stored into the other buffer (one
-  // barrier per chunk)
-  __shared__ __align__(16) float As[2 * CHF];
-  __shared__ int s_class, s_start, s_n;
-  const int tid = threadIdx.x;
-  int cls0, split, tile;
-  if (region) {
-    const int xcd = blockIdx.x & 7, item = blockIdx.x >> 3, tpr = (int)(gridDim.x >> 6) / nsplit;
-    cls0 = item & 7;
-    split = (item >> 3) % nsplit;
-    tile = xcd * tpr + (item >> 3) / nsplit;
-  } else {
-    const int item = blockIdx.x >> 3, tpc = (int)(gridDim.x >> 3) / nsplit;
-    cls0 = blockIdx.x & 7;
-    split = item / tpc;
-    tile = item % tpc;
-  }
-  if (tid == 0) {
-    int start = 0;
-    for (int c = 0; c < cls0; c++) start += cls_cnt[c];
-    const int cnt = cls_cnt[cls0], nt = (cnt + TN - 1) / TN;
-    s_class = tile < nt ? cls0 : -1;
-    s_start = start + tile * TN;
-    s_n = tile < nt ? min(TN, cnt - tile * TN) : 0;
-  }
-  __syncthreads();
-  const int cls = s_class, ntile = s_n;
-  if (cls < 0) return;
-  const int w = tid >> 6, l = tid & 63, j = l & 15, kq = l >> 4;
-  const int g = 1 << lev;
-  const int t = w * 16 + j;
-  int tord = -1, tx = 0, ty = 0, tz = 0;
-  if (t < ntile) {
-    tord = (int)ord[s_start + t];
-    morton_decode(ikey[tord], lev, tx, ty, tz);
-  }
-  const bool wave_on = w * 16 < ntile;
-  const int per = (NEBM + nsplit - 1) / nsplit, o0 = split * per, o1 = min(NEBM, o0 + per);
-  V4 acc[MT];
-#pragma unroll
-  for (int mt = 0; mt < MT; mt++) acc[mt] = V4{0.f, 0.f, 0.f, 0.f};
-  unsigned long long mypairs = 0;
-  // lane kq holds k = kq KS + ks: part kq / 2, slots (kq % 2) KS + ks
-  const int bpart = kq >> 1, bslot = (kq & 1) * KS;
-  constexpr int NV4 = (CHF / 4 + NTH - 1) / NTH;  // float4 per thread per chunk
-  V4 areg[NV4];
-#define FMMX_HH_OP(o_) (opF + (size_t)(offtab[cls * NEBM + (o_)].w & 0xffff) * FR)
-#define FMMX_HH_LOAD(a_, c_)                                                                     \
-  {                                                                                              \
-    const int nf4_ = min(HH_KC, KS - (c_) * HH_KC) * MT * 16;                                     \
-    const V4* src_ = reinterpret_cast<const V4*>((a_) + (size_t)(c_) * CHF);             \
-    _Pragma("unroll") for (int v = 0; v < NV4; v++) {                                            \
-      const int e_ = tid + NTH * v;                                                              \
-      if (e_ < nf4_) areg[v] = src_[e_];                                                         \
-    }                                                                                            \
-  }
-#define FMMX_HH_STORE(buf_, c_)                                                                  \
-  {                                                                                              \
-    const int nf4_ = min(HH_KC, KS - (c_) * HH_KC) * MT * 16;                                     \
-    V4* dst_ = reinterpret_cast<V4*>(As + (buf_) * CHF);                                 \
-    _Pragma("unroll") for (int v = 0; v < NV4; v++) {                                            \
-      const int e_ = tid + NTH * v;                                                              \
-      if (e_ < nf4_) dst_[e_] = areg[v];                                                         \
-    }                                                                                            \
-  }
-  if (o0 < o1) {
-    FMMX_HH_LOAD(FMMX_HH_OP(o0), 0);
-    FMMX_HH_STORE(0, 0);
-  }
-  __syncthreads();
-  int buf = 0;
-  for (int o = o0; o < o1; o++) {
-    const int4 off = offtab[cls * NEBM + o];
-    int s_ = -1;
-    if (tord >= 0) {
-      const int jx = tx - off.x, jy = ty - off.y, jz = tz - off.z;
-      if (jx >= 0 && jx < g && jy >= 0 && jy < g && jz >= 0 && jz < g &&
-          (gsh < 0 || !((jx ^ tx) >> gsh | (jy ^ ty) >> gsh | (jz ^ tz) >> gsh)))
-        s_ = dense_j[morton_encode(jx, jy, jz, lev)];
-    }
-    if (s_ >= 0 && kq == 0) mypairs++;
-    const bool any = wave_on && __ballot(s_ >= 0) != 0;
-    float b[KS];
-    if (any) {
-      const float* ms = M + (size_t)(s_ >= 0 ? s_ : 0) * 2 * ML::VS + bpart * ML::VS;
-#pragma unroll
-      for (int ks = 0; ks < KS; ks++) b[ks] = s_ >= 0 ? ms[ML::at(bslot + ks)] : 0.f;
-    }
-    const float* Acur = FMMX_HH_OP(o);
-    const float* Anext = o + 1 < o1 ? FMMX_HH_OP(o + 1) : nullptr;
-#pragma unroll
-    for (int c = 0; c < NCH; c++) {
-      // the next chunk: of this offset, or the first of the next offset
-      const bool has_next = c + 1 < NCH || Anext != nullptr;
-      if (c + 1 < NCH) FMMX_HH_LOAD(Acur, c + 1)
-      else if (Anext) FMMX_HH_LOAD(Anext, 0)
-      if (any) {
-        const float* Ab = As + buf * CHF;
-#pragma unroll
-        for (int kk = 0; kk < HH_KC; kk++) {
-          const int ks = c * HH_KC + kk;
-          if (ks < KS) {
-            float af[MT];
-#pragma unroll
-            for (int mt = 0; mt < MT; mt++) af[mt] = Ab[(kk * MT + mt) * 64 + l];
-#pragma unroll
-            for (int mt = 0; mt < MT; mt++) acc[mt] = Mfma<float>::fma(af[mt], b[ks], acc[mt]);
-          }
-        }
-      }
-      if (has_next) FMMX_HH_STORE(buf ^ 1, c + 1 < NCH ? c + 1 : 0)
-      __syncthreads();
-      buf ^= 1;
-    }
-  }
-#undef FMMX_HH_OP
-#undef FMMX_HH_LOAD
-#undef FMMX_HH_STORE
-  if (tord >= 0) {
-#pragma unroll
-    for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int i = 16 * mt + 4 * kq + r;
-        if (i < D) {
-          const float v = acc[mt][r];
-          if (nsplit == 1) {
-            float* dst = L + (size_t)tord * D + i;
-            *dst = init ? v : *dst + v;
-          } else {
-            part[((size_t)split * nb + tord) * D + i] = v;
-          }
-        }
-      }
-  }
-  if (mypairs) atomicAdd(npairs, mypairs);
-}
-
 // FP64 M2L on the vector FMA units (MI355X: FP64 vector peak = FP64 matrix
 // peak).  Same tiles and offset split as k_m2l; per offset the operator
 // (k-major) and the gathered source multipoles go through LDS in K-chunks
@@ -739,6 +576,10 @@ Engine::M2LVariant Engine::m2l_variant(int lev) const {
       // 0.331 ms for the launch, 16 splits 0.341; a sphere's leaf level of
       // 4,639 boxes 0.104 against 0.125)
       if (v.pa == 6 && tpc > 1) v.nsplit = std::min(v.nsplit, 8);
+      // Helmholtz: one workgroup per CU and 1.5 KB of partial sums per target
+      // and split (sphere of 1M points: 4 splits of the leaf level 1.68 ms for
+      // M2L and L2L, 7 splits 1.84, 2 splits 1.85)
+      if (hh) v.nsplit = std::max(1, std::min(640 / (8 * tpc), tpc > 1 ? 8 : 16));
     }
   }
   v.nsplit = std::max(1, std::min(16, v.nsplit));
@@ -851,6 +692,7 @@ int Engine::run_msplit(int l0, int l1, int form) {
 // the L2L chain then adds the parents' locals level by level.  With the FP16
 // split shape (staging 3, 4) the multipoles are split first.
 int Engine::run_m2l_all(int l0) {
+  if (hh) return run_m2l_hh(l0, lmax, true);
   const M2LVariant leaf = m2l_variant(lmax);
   const bool split = leaf.pa >= 3, orbit = leaf.pa == 6;
   // floats of a target's partial sums (the orbit form always goes through them)
@@ -921,9 +763,49 @@ int Engine::run_m2l_all(int l0) {
   });
 }
 
+// FP32 Helmholtz M2L of levels l0..l1 by reflection orbits, one launch; the
+// locals are written (init) or added to
+int Engine::run_m2l_hh(int l0, int l1, bool init) {
+  M2LLaunch A{};
+  MSplitLevels S{};
+  const size_t rows = orbit_gen_rows(p, 1), frg = orbit_gen_frags(p, 1);
+  size_t need = 0;
+  for (int lev = l0; lev <= l1; lev++)
+    if (si.nb[lev] > 0 && sj.nb[lev] > 0) need += (size_t)m2l_splits(lev) * si.nb[lev] * rows;
+  int rc = m2l_part.ensure(std::max<size_t>(need, 1) * 4);
+  if (rc || (rc = mmax_buf.ensure((MAXL + 1) * 4))) return rc;
+  size_t off = 0;
+  int wg = 0;
+  for (int lev = l0; lev <= l1; lev++) {
+    const int nb = si.nb[lev];
+    if (nb == 0) continue;
+    if (sj.nb[lev] == 0) {
+      const long nl = (long)nb * P2 * 2;
+      if (init) k_zero_t<float><<<(int)((nl + 255) / 256), 256, 0, stream>>>(nl, lexp[lev].as<float>());
+      continue;
+    }
+    S.M[S.nl] = mexp[lev].as<float>();
+    S.Mh[S.nl] = mexp_h[lev].as<uint4>();
+    S.mmax[S.nl] = mmax_buf.as<unsigned>() + lev;
+    S.off[S.nl + 1] = S.off[S.nl] + sj.nb[lev] + 1;
+    S.nl++;
+    const int ns = m2l_splits(lev);
+    M2LLev& d = A.lv[A.nlv++] = m2l_desc(lev, 1, ORB_WPG, ns, m2l_part.as<float>() + off, init ? 1 : 0, wg);
+    d.opH = hop_m2l.as<uint4>() + (size_t)(lev - 2) * NORBOP * frg;
+    d.sa_e = hop_e[lev];
+    wg += d.nwg;
+    off += (size_t)ns * nb * rows;
+  }
+  if (A.nlv == 0) return FMMX_OK;
+  if ((rc = launch_orbit_gen_order(p, 1, S, stream))) return rc;
+  if ((rc = launch_m2l_orbit_gen(p, 1, A, wg, orbtab.as<int4>(), stream))) return rc;
+  return launch_orbit_gen_reduce(p, 1, A, stream);
+}
+
 int Engine::run_m2l(int lev, bool init, int phase) {
   const int nb = si.nb[lev];
   if (nb == 0) return FMMX_OK;
+  if (hh && !fp64) return run_m2l_hh(lev, lev, init);
   const long nl = (long)nb * P2 * parts();
   if (sj.nb[lev] == 0) {
     if (init && phase != 1) {
@@ -962,38 +844,18 @@ int Engine::run_m2l(int lev, bool init, int phase) {
 
   const int gsh = group_shift(lev);
   if (hh) {
-    // split complex expansions: D = 2 p^2, k-major operators per level, on the
-    // vector units in both precisions
+    // FP64: split complex expansions, D = 2 p^2, k-major operators per level, on
+    // the vector units
     const size_t hoff = (size_t)(lev - 2) * NOFF * 4 * P2 * P2;
     return dispatch_hp(p, [&](auto pc) -> int {
       constexpr int P = decltype(pc)::value;
-      if (fp64)
-        k_m2l_vec<P, double, 2><<<tiles * nsplit, 256, 0, stream>>>(
-            lev, nb, nsplit, cls_cnt[lev].as<int>(), cls_ord[lev].as<uint32_t>(), si.bkey[lev].as<uint32_t>(),
-            sj.dense[lev].as<int>(), mexp[lev].as<double>(), lexp[lev].as<double>(), part_buf->as<double>(),
-            hop_m2l.as<double>() + hoff, offtab.as<int4>(), init ? 1 : 0, gsh, pair_ctr.as<unsigned long long>() + 2 + lev);
-      else {
-        // MFMA, 8 waves of 16 targets per workgroup, operator chunks in LDS
-        constexpr int D = 2 * P * P, FRH = (D / 4) * ((D + 15) / 16) * 64;
-        int cmax = 0;
-        for (int c = 0; c < 8; c++) cmax = std::max(cmax, cls_cnt_h[lev][c]);
-        const int tpc = std::max(1, (cmax + 127) / 128);
-        const int region = tpc >= 8 ? 1 : 0;
-        const int nwg = region ? 64 * ((tpc + 7) / 8) * nsplit : 8 * tpc * nsplit;
-        k_m2l_hh<P, 8><<<nwg, 512, 0, stream>>>(
-            lev, nb, nsplit, cls_cnt[lev].as<int>(), cls_ord[lev].as<uint32_t>(), si.bkey[lev].as<uint32_t>(),
-            sj.dense[lev].as<int>(), mexp[lev].as<float>(), lexp[lev].as<float>(), part_buf->as<float>(),
-            hop_m2l.as<float>() + (size_t)(lev - 2) * NOFF * FRH, offtab.as<int4>(), init ? 1 : 0, region, gsh,
-            pair_ctr.as<unsigned long long>() + 2 + lev);
-      }
-      if (nsplit > 1 && phase == 0) {
-        if (fp64)
-          k_m2l_reduce<double><<<(int)((nl + 255) / 256), 256, 0, stream>>>(nl, nsplit, part_buf->as<double>(),
-                                                                            lexp[lev].as<double>(), init ? 1 : 0);
-        else
-          k_m2l_reduce<float><<<(int)((nl + 255) / 256), 256, 0, stream>>>(nl, nsplit, part_buf->as<float>(),
-                                                                           lexp[lev].as<float>(), init ? 1 : 0);
-      }
+      k_m2l_vec<P, double, 2><<<tiles * nsplit, 256, 0, stream>>>(
+          lev, nb, nsplit, cls_cnt[lev].as<int>(), cls_ord[lev].as<uint32_t>(), si.bkey[lev].as<uint32_t>(),
+          sj.dense[lev].as<int>(), mexp[lev].as<double>(), lexp[lev].as<double>(), part_buf->as<double>(),
+          hop_m2l.as<double>() + hoff, offtab.as<int4>(), init ? 1 : 0, gsh, pair_ctr.as<unsigned long long>() + 2 + lev);
+      if (nsplit > 1 && phase == 0)
+        k_m2l_reduce<double><<<(int)((nl + 255) / 256), 256, 0, stream>>>(nl, nsplit, part_buf->as<double>(),
+                                                                          lexp[lev].as<double>(), init ? 1 : 0);
       FMMX_HIP(hipGetLastError());
       return FMMX_OK;
     });

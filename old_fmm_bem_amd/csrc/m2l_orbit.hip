@@ -8,32 +8,11 @@
 // per target instead of 189.  The transformed sources are then carried as FP16
 // hi + lo against hi + lo operators (three products, FP32 accumulation), as in
 // m2l_split.hip.
-#include <type_traits>
-
-#include "m2l.h"
-#include "tree_util.h"
+#include "orbit.h"
 
 namespace fmmx {
 
 namespace {
-
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
-// 2^e that brings the level's largest magnitude just below 2^ORB_TOP
-__device__ __forceinline__ int orbit_exp(const unsigned* mmax) {
-  const float m = __uint_as_float(*mmax);
-  if (!(m > 0.f) || !(m < 3.0e38f)) return 0;
-  int e;
-  (void)frexpf(m, &e);
-  return min(100, max(-100, ORB_TOP - e));
-}
-
-// bits of v (0..3) at positions 0 and 3 (one axis of a Morton key)
-__device__ __forceinline__ uint32_t dil3(int v) { return (uint32_t)(v & 1) | ((uint32_t)(v & 2) << 2); }
 
 // stored position of every float of an orbit box in the padded multipole
 // layout (-1: zero), and the partial-sum position of every local slot
@@ -74,40 +53,6 @@ __global__ __launch_bounds__(256) void k_morder(MSplitLevels S) {
   if (b != S.off[k + 1] - 1 && src >= 0)
     v = S.M[k][(size_t)(b - S.off[k]) * MLayout<P>::VS + src] * ldexpf(1.f, orbit_exp(S.mmax[k]));
   reinterpret_cast<float*>(S.Mh[k])[(size_t)(b - S.off[k]) * OC::BS + e] = v;
-}
-
-// rank of a submask of D among the submasks (pext)
-constexpr __host__ __device__ int sub_rank(int D, int r) {
-  int s = 0, j = 0;
-  for (int a = 0; a < 3; a++)
-    if ((D >> a) & 1) s |= ((r >> a) & 1) << j++;
-  return s;
-}
-constexpr __host__ __device__ int bits3(int D) { return (D & 1) + ((D >> 1) & 1) + ((D >> 2) & 1); }
-// in-place Walsh-Hadamard transform over the 2^J sources of one word
-template <int J>
-__device__ __forceinline__ void wht(float (&raw)[1 << J][4], int t) {
-#pragma unroll
-  for (int b = 0; b < J; b++)
-#pragma unroll
-    for (int s = 0; s < (1 << J); s++)
-      if (!(s & (1 << b))) {
-        const float u = raw[s][t], v = raw[s | (1 << b)][t];
-        raw[s][t] = u + v;
-        raw[s | (1 << b)][t] = u - v;
-      }
-}
-
-__device__ __forceinline__ uint32_t hi_pair(float a, float b) {
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, h2));
-}
-// the residuals of a pair against its rounded halves h (exact in FP32:
-// a - h in one mixed fused multiply-add)
-__device__ __forceinline__ uint32_t lo_pair(float a, float b, uint32_t h) {
-  float ra, rb;
-  asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(ra) : "v"(h), "v"(a));
-  asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(rb) : "v"(h), "v"(b));
-  return hi_pair(ra, rb);
 }
 
 constexpr int ORB_NTH = 64 * ORB_WPG, ORB_TN = 16 * ORB_WPG;
