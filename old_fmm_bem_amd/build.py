@@ -28,7 +28,7 @@ COMMON = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-I" + os.path
 
 CORE = ["precompute.cpp", "yukawa.cpp", "helmholtz.cpp", "split_host.cpp", "tree.hip", "p2m.hip",
         "l2p.hip", "translate.hip", "m2l.hip", "p2p.hip", "m2l_split.hip",
-        "m2l_orbit.hip", "m2l_orbit_gen.hip", "api.cpp", "adjoint.cpp"]
+        "m2l_orbit.hip", "m2l_orbit_gen.hip", "m2l_orbit_fp64.hip", "api.cpp", "adjoint.cpp"]
 SHIM = ["refshim.cpp"]
 
 

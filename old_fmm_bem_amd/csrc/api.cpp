@@ -198,6 +198,7 @@ struct OpSet {
   std::vector<uint4> m2l_wide;
   // the same split for the reflection-orbit kernel: its NORBOP operators
   std::vector<uint4> m2l_orbit;
+  std::vector<double> m2l_orbit_f64;  // the orbit operators of the FP64 engine (get_orbit_f64)
   std::vector<int> lev_e;  // scale exponents of per-level orbit operators
   int nlev = 1;
 };
@@ -314,6 +315,13 @@ std::shared_ptr<OpSet> get_ops(const Tables& T, int lmax, float rd) {
   std::lock_guard<std::mutex> lk(g_cache_mu);
   g_cache[key] = S;
   return S;
+}
+
+// the FP64 orbit fragments of a Laplace set, built when an FP64 engine first asks
+const std::vector<double>& get_orbit_f64(OpSet& S, int p) {
+  std::lock_guard<std::mutex> lk(g_cache_mu);
+  if (S.m2l_orbit_f64.empty()) orbit_f64_fragments(S.m2l_kmaj.data(), p, S.m2l_orbit_f64);
+  return S.m2l_orbit_f64;
 }
 
 // Yukawa operator sets keyed by (p, lambda, rd, lmax): M2M per parent level
@@ -718,7 +726,8 @@ int Engine::upload_yukawa_operators() {
   auto S = get_yuk_ops(p, lam, rd, lmax);
   int rc;
   if (fp64) {
-    if ((rc = upload<double>(yop_m2m, S->m2m, stream)) || (rc = upload<double>(yop_l2l, S->l2l, stream)) ||
+    if ((rc = upload<double>(yop_m2m, p > P_ALL ? S->m2m : S->m2m_frag, stream)) ||
+        (rc = upload<double>(yop_l2l, p > P_ALL ? S->l2l : S->l2l_frag, stream)) ||
         (rc = upload<double>(yop_m2l, S->m2l_kmaj, stream)))
       return rc;
   } else {
@@ -738,8 +747,11 @@ int Engine::upload_operators() {
   m2l_per_level = S->nlev > 1;
   int rc;
   if (fp64) {
-    if ((rc = upload<double>(op_m2m, S->m2m, stream)) || (rc = upload<double>(op_l2l, S->l2l, stream)) ||
-        (rc = upload<double>(op_m2l, S->m2l_kmaj, stream)))
+    orb64_ok = cfg.convention == FMMX_CONV_EXACT && orbit_f64_supported(p);
+    if ((rc = upload<double>(op_m2m, p > P_ALL ? S->m2m : S->m2m_frag, stream)) ||
+        (rc = upload<double>(op_l2l, p > P_ALL ? S->l2l : S->l2l_frag, stream)) ||
+        (rc = orb64_ok ? upload<double>(op_m2l_of, get_orbit_f64(*S, p), stream)
+                       : upload<double>(op_m2l, S->m2l_kmaj, stream)))
       return rc;
   } else {
     if ((rc = upload<float>(op_m2m, S->m2m_frag, stream)) || (rc = upload<float>(op_l2l, S->l2l_frag, stream)) ||
@@ -964,6 +976,7 @@ int Engine::prepare(int neq) {
         (rc = lexp[l].ensure((size_t)std::max(1, si.nb[l]) * P2 * np * es)))
       return rc;
     if (hh && !fp64 && (rc = mexp_h[l].ensure((size_t)(sj.nb[l] + 1) * orbit_gen_box_floats(p, 1) * 4))) return rc;
+    if (orbit_f64() && (rc = mexp_h[l].ensure((size_t)(sj.nb[l] + 1) * orbit_f64_box(p) * 8))) return rc;
     if (split_ok && !hh && !fp64 && (rc = mexp_h[l].ensure((size_t)(sj.nb[l] + 1) * split_box_halfs(p) * 2)))
       return rc;
   }

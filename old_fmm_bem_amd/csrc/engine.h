@@ -218,6 +218,8 @@ struct Engine {
 
   int hop_e[MAXL + 1] = {};  // scale exponents of hop_m2l per level (FP32)
 
+  DevBuf op_m2l_of;       // FP64 orbit operators (op_m2l is not uploaded with them)
+  bool orb64_ok = false;
   ~Engine();
   int init(const fmmx_config* c, int dev, void* stream);
   int set_points(int ni, const float* xi, const float* yi, const float* zi, const float* nxi, const float* nyi,
@@ -266,13 +268,16 @@ struct Engine {
   M2LVariant m2l_variant(int lev) const;
   int m2l_splits(int lev) const { return m2l_variant(lev).nsplit; }
   int run_m2l(int lev, bool init, int phase = 0);
-  int run_m2l_all(int l0);  // FP32: every level in one launch
+  int run_m2l_all(int l0);  // every level in one launch (FP32; FP64 by orbits)
   int run_m2l_hh(int l0, int l1, bool init);  // FP32 Helmholtz, levels l0..l1 in one launch
+  int run_m2l_f64(int l0, int l1, bool init);  // FP64 by reflection orbits, levels l0..l1 in one launch
+  // the FP64 form by reflection orbits: Laplace, EXACT, p = 6..12 (m2l_orbit_fp64.hip)
+  bool orbit_f64() const { return fp64 && orb64_ok && !yk && !hh; }
   int run_msplit(int l0, int l1, int form);  // split multipoles for the FP16 kernels
   bool last_m2l_all = false;  // the last evaluation took that form
   bool m2l_timed = false;     // the last evaluation recorded ev[8], ev[9] around its M2L launch
   bool m2l_all_levels() const {
-    if (fp64) return false;
+    if (fp64) return orbit_f64();
     const char* e = getenv("FMMX_M2L_FUSED");
     return !e || atoi(e) != 0;
   }
@@ -290,20 +295,20 @@ struct Engine {
   // (pi/2)/lambda of kernel/Helmholtz_G_p2p.cxx:22 (float pi in REF)
   double c_yukawa() const { return (cfg.convention == FMMX_CONV_REF ? 0.5 * (double)PIF : 0.5 * M_PI) / lam; }
   // translation operators of the evaluation in progress
-  // (FP32 Laplace and Yukawa: MFMA fragment order, FR floats per octant)
+  // (Laplace and Yukawa up to P_ALL: MFMA fragment order, FR values per octant)
   size_t frag_size() const { return (size_t)((P2 + 3) / 4) * ((P2 + 15) / 16) * 64; }
   template <class T>
   const T* m2m_ops(int parent_lev) const {
     if (hh && fp64) return hop_m2m.as<T>() + (size_t)(parent_lev - 2) * 8 * 4 * VS * VS;
     if (hh) return hop_m2m.as<T>() + (size_t)(parent_lev - 2) * 8 * frag_size();
-    const size_t per = fp64 ? (size_t)VS * VS : frag_size();
+    const size_t per = p > P_ALL ? (size_t)VS * VS : frag_size();
     return yk ? yop_m2m.as<T>() + (size_t)(parent_lev - 2) * 8 * per : op_m2m.as<T>();
   }
   template <class T>
   const T* l2l_ops(int child_lev) const {
     if (hh && fp64) return hop_l2l.as<T>() + (size_t)(child_lev - 3) * 8 * 4 * P2 * P2;
     if (hh) return hop_l2l.as<T>() + (size_t)(child_lev - 3) * 8 * frag_size();
-    const size_t per = fp64 ? (size_t)P2 * P2 : frag_size();
+    const size_t per = p > P_ALL ? (size_t)P2 * P2 : frag_size();
     return yk ? yop_l2l.as<T>() + (size_t)(child_lev - 3) * 8 * per : op_l2l.as<T>();
   }
   double rb(int lev) const { return (double)rd / (double)(1 << lev); }

@@ -225,6 +225,34 @@ struct GConst {
   static constexpr int CH = NT * PARTS * 2 * 64, FRO = NSTEP * CH;  // 16-byte fragments of a step, operator
   static constexpr int ROWS = PARTS * NT * 16;                      // partial sums per target
 };
+// The FP64 form (m2l_orbit_fp64.hip) in the general layout: k-step ks takes one
+// word of a class (4 members), two k-steps share a lane's 16-byte word and
+// fragment, and the last octet ends with its last word that any class has.
+template <int P>
+struct FConst {
+  static constexpr GLayout<P> L{};
+  static constexpr int NO = L.no, XTRA = L.xtra, NSTEP = NO + XTRA, NT = L.nt;
+  static constexpr bool two() {
+    for (int k = 0; k < 8; k++)
+      if (L.O.size[k] > 4 * NO + 4) return true;
+    return false;
+  }
+  static constexpr int NKX = XTRA ? (two() ? 8 : 4) : 0, NKS = 8 * NO + NKX;  // k-steps of the last octet, of all
+  static constexpr int NU = NKS / 2, BS = NU * 8;                   // 64-byte units, doubles of a stored box
+  static constexpr int CH = 4 * NT * 64, CHX = NKX / 2 * NT * 64;   // 16-byte fragments of an octet, the last one
+  static constexpr int FRO = NO * CH + CHX, ROWS = NT * 16;         // fragments of an operator, partial sums per target
+  // step of a k-step and its place in it
+  static constexpr __host__ __device__ int step(int ks) { return ks / 8; }
+  static constexpr __host__ __device__ int place(int ks) { return ks % 8; }
+};
+inline bool orbit_f64_supported(int p) { return p >= 6 && p <= P_ALL; }
+int launch_m2l_orbit_f64(int p, const MSplitLevels& S, const M2LLaunch& A, int nwg, const int4* orbtab, hipEvent_t e0,
+                         hipEvent_t e1, hipStream_t stream);
+size_t orbit_f64_box(int p);   // doubles of a stored box
+size_t orbit_f64_rows(int p);  // partial sums per target
+// fragments of the NORBOP operators from all 316 k-major ones
+void orbit_f64_fragments(const double* kmaj, int p, std::vector<double>& out);
+
 // launchers of the general form; opset[lev]: fragments of that level's operators
 int launch_m2l_orbit_gen(int p, int hh, const M2LLaunch& A, int nwg, const int4* orbtab, hipStream_t stream);
 int launch_orbit_gen_order(int p, int hh, const MSplitLevels& S, hipStream_t stream);

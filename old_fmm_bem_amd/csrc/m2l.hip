@@ -351,8 +351,9 @@ __global__ __launch_bounds__(64 * WPG) void k_m2l(M2LLaunch A) {
   if (mypairs) atomicAdd(npairs, mypairs);
 }
 
-// FP64 M2L on the vector FMA units (MI355X: FP64 vector peak = FP64 matrix
-// peak).  Same tiles and offset split as k_m2l; per offset the operator
+// FP64 M2L on the vector FMA units, for what the orbit form (m2l_orbit_fp64.hip)
+// is not built for: the REF convention, orders below 6 and 18, the Yukawa and
+// Helmholtz kernels.  Same tiles and offset split as k_m2l; per offset the operator
 // (k-major) and the gathered source multipoles go through LDS in K-chunks
 // and each thread accumulates a (rows x 4 targets) register block.
 constexpr int M2LV_KC = 32, M2LV_BST = M2L_TN + 4;
@@ -563,7 +564,7 @@ Engine::M2LVariant Engine::m2l_variant(int lev) const {
   }
   if (v.nsplit <= 0) {
     // enough workgroups to cover the chip: split the 189 offsets when tiles are few
-    if (fp64) {
+    if (fp64 && !orbit_f64()) {
       v.nsplit = 1024 / ((si.nb[lev] + M2L_TN - 1) / M2L_TN + 8);
     } else {
       int cmax = 0;
@@ -579,6 +580,9 @@ Engine::M2LVariant Engine::m2l_variant(int lev) const {
       // Helmholtz: one workgroup per CU and 1.5 KB of partial sums per target
       // and split (sphere of 1M points: 4 splits of the leaf level 1.68 ms for
       // M2L and L2L, 7 splits 1.84, 2 splits 1.85)
+      // FP64 orbits: 512 workgroups of a level, each with its own share of the
+      // 63 products (one workgroup per CU at a time)
+      if (orbit_f64()) v.nsplit = 512 / (8 * tpc);
       if (hh) v.nsplit = std::max(1, std::min(640 / (8 * tpc), tpc > 1 ? 8 : 16));
     }
   }
@@ -693,6 +697,7 @@ int Engine::run_msplit(int l0, int l1, int form) {
 // split shape (staging 3, 4) the multipoles are split first.
 int Engine::run_m2l_all(int l0) {
   if (hh) return run_m2l_hh(l0, lmax, true);
+  if (fp64) return run_m2l_f64(l0, lmax, true);
   const M2LVariant leaf = m2l_variant(lmax);
   const bool split = leaf.pa >= 3, orbit = leaf.pa == 6;
   // floats of a target's partial sums (the orbit form always goes through them)
@@ -802,10 +807,49 @@ int Engine::run_m2l_hh(int l0, int l1, bool init) {
   return launch_orbit_gen_reduce(p, 1, A, stream);
 }
 
+// FP64 Laplace M2L of levels l0..l1 by reflection orbits, one launch; the locals
+// are written (init) or added to
+int Engine::run_m2l_f64(int l0, int l1, bool init) {
+  M2LLaunch A{};
+  MSplitLevels S{};
+  const size_t rows = orbit_f64_rows(p);
+  size_t need = 0;
+  for (int lev = l0; lev <= l1; lev++)
+    if (si.nb[lev] > 0 && sj.nb[lev] > 0) need += (size_t)m2l_splits(lev) * si.nb[lev] * rows;
+  int rc = m2l_part.ensure(std::max<size_t>(need, 1) * 8);
+  if (rc) return rc;
+  size_t off = 0;
+  int wg = 0;
+  for (int lev = l0; lev <= l1; lev++) {
+    const int nb = si.nb[lev];
+    if (nb == 0) continue;
+    if (sj.nb[lev] == 0) {
+      const long nl = (long)nb * P2;
+      if (init) k_zero_t<double><<<(int)((nl + 255) / 256), 256, 0, stream>>>(nl, lexp[lev].as<double>());
+      continue;
+    }
+    S.M[S.nl] = mexp[lev].as<float>();
+    S.Mh[S.nl] = mexp_h[lev].as<uint4>();
+    S.off[S.nl + 1] = S.off[S.nl] + sj.nb[lev] + 1;
+    S.nl++;
+    const int ns = m2l_splits(lev);
+    float* part = reinterpret_cast<float*>(m2l_part.as<double>() + off);
+    M2LLev& d = A.lv[A.nlv++] = m2l_desc(lev, 1, ORB_WPG, ns, part, init ? 1 : 0, wg);
+    d.opH = op_m2l_of.as<uint4>();
+    wg += d.nwg;
+    off += (size_t)ns * nb * rows;
+  }
+  if (A.nlv == 0) return FMMX_OK;
+  const bool tmark = per_phase && l1 == lmax;
+  m2l_timed = m2l_timed || tmark;
+  return launch_m2l_orbit_f64(p, S, A, wg, orbtab.as<int4>(), tmark ? ev[8] : nullptr, tmark ? ev[9] : nullptr, stream);
+}
+
 int Engine::run_m2l(int lev, bool init, int phase) {
   const int nb = si.nb[lev];
   if (nb == 0) return FMMX_OK;
   if (hh && !fp64) return run_m2l_hh(lev, lev, init);
+  if (orbit_f64()) return run_m2l_f64(lev, lev, init);
   const long nl = (long)nb * P2 * parts();
   if (sj.nb[lev] == 0) {
     if (init && phase != 1) {

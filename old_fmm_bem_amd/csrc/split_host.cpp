@@ -276,4 +276,48 @@ void orbit_gen_fragments(const double* C, const double* S, int ld, int p, int sa
   }
 }
 
+namespace {
+template <typename G>
+auto with_f64(int p, G&& f) {
+  switch (p) {
+#define FMMX_CASE(P) \
+  case P:            \
+    return f(std::integral_constant<int, P>{});
+    FMMX_CASE(6) FMMX_CASE(7) FMMX_CASE(8) FMMX_CASE(9) FMMX_CASE(10) FMMX_CASE(11)
+#undef FMMX_CASE
+  }
+  return f(std::integral_constant<int, 12>{});
+}
+}  // namespace
+
+size_t orbit_f64_box(int p) {
+  return with_f64(p, [](auto pc) -> size_t { return FConst<decltype(pc)::value>::BS; });
+}
+size_t orbit_f64_rows(int p) {
+  return with_f64(p, [](auto pc) -> size_t { return FConst<decltype(pc)::value>::ROWS; });
+}
+void orbit_f64_fragments(const double* kmaj, int p, std::vector<double>& out) {
+  with_f64(p, [&](auto pc) {
+    constexpr int P = decltype(pc)::value, P2 = P * P;
+    using F = FConst<P>;
+    constexpr GLayout<P> L{};
+    const auto& ops = orbit_ops();
+    out.assign((size_t)NORBOP * F::FRO * 2, 0.0);
+    for (size_t oi = 0; oi < ops.size(); oi++) {
+      const double* A = kmaj + (size_t)offset_index(ops[oi][0], ops[oi][1], ops[oi][2]) * P2 * P2;  // (i, k) at [k P2 + i]
+      double* dst = &out[oi * F::FRO * 2];
+      for (int ks = 0; ks < F::NKS; ks++)
+        for (int tl = 0; tl < F::NT; tl++)
+          for (int l = 0; l < 64; l++) {
+            // row rho of v_mfma_f64_16x16x4 comes out in lane group rho % 4, register rho / 4
+            const int r = L.trow[tl] + 4 * (l & 3) + ((l & 15) >> 2);
+            const int m = L.member(F::step(ks), F::place(ks), l >> 4);
+            if (m < 0 || r >= L.O.size[L.tcls[tl]]) continue;
+            const int i = L.O.slot[L.tcls[tl]][r], k = L.O.slot[L.cls(F::step(ks), F::place(ks))][m];
+            dst[(((size_t)ks / 2 * F::NT + tl) * 64 + l) * 2 + (ks & 1)] = A[(size_t)k * P2 + i];
+          }
+    }
+  });
+}
+
 }  // namespace fmmx

@@ -126,7 +126,7 @@ __global__ __launch_bounds__(TR_NT) void k_translate(int nout, const int* __rest
 }
 
 // ---------------------------------------------------------------------
-// M2M and L2L of the FP32 engine on MFMA (v_mfma_f32_16x16x4f32), operators
+// M2M and L2L on MFMA (v_mfma_f32_16x16x4f32, v_mfma_f64_16x16x4f64), operators
 // in the fragment order of the M2L kernel ([ks][mt][lane] holds row
 // 16 mt + lane % 16, column (lane / 16) KS + ks of the p^2 x p^2 operator).
 //   M2M: a workgroup of 8 waves owns 16 parent boxes; wave w multiplies the
@@ -143,19 +143,23 @@ __global__ __launch_bounds__(TR_NT) void k_translate(int nout, const int* __rest
 // re-expansions do not mix them); blockIdx.y is the part.  Helmholtz at p = 12
 // on a sphere of 1M points (lmax 6), M2M and L2L of all levels: 1.41 + 1.15 ms
 // as (2 p^2)^2 products on the vector units, 0.142 + 0.135 ms here.
-template <int P, int L2L>
+// FP64 (the same fragments in double; a lane's output rows are 4 r + l / 16
+// instead of 4 (l / 16) + r): 4,096 children at p = 10 24 + 23 us against 48 + 43
+// us for one M2M and L2L level in k_translate, whose FMAs wait for LDS.
+template <int P, int L2L, typename T>
 __global__ __launch_bounds__(L2L ? 256 : 512) void k_translate_mfma(int nout, const int* __restrict__ cfirst,
                                                                     const uint32_t* __restrict__ key,
                                                                     const int* __restrict__ parent,
                                                                     const int* __restrict__ cls_cnt,
                                                                     const uint32_t* __restrict__ ord,
-                                                                    const float* __restrict__ in,
-                                                                    float* __restrict__ out,
-                                                                    const float* __restrict__ opF, int add,
+                                                                    const T* __restrict__ in,
+                                                                    T* __restrict__ out,
+                                                                    const T* __restrict__ opF, int add,
                                                                     int parts) {
   using ML = MLayout<P>;
   constexpr int P2 = P * P, MT = (P2 + 15) / 16, KS = (P2 + 3) / 4, FR = KS * MT * 64;
-  using V4 = f32x4;
+  using V4 = typename Mfma<T>::v4;
+  constexpr bool D = sizeof(T) == 8;
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, j = l & 15, kq = l >> 4;
   in += (size_t)blockIdx.y * (L2L ? P2 : ML::VS);
   out += (size_t)blockIdx.y * (L2L ? P2 : ML::VS);
@@ -188,32 +192,32 @@ __global__ __launch_bounds__(L2L ? 256 : 512) void k_translate_mfma(int nout, co
   }
   V4 acc[MT];
 #pragma unroll
-  for (int mt = 0; mt < MT; mt++) acc[mt] = V4{0.f, 0.f, 0.f, 0.f};
+  for (int mt = 0; mt < MT; mt++) acc[mt] = V4{T(0), T(0), T(0), T(0)};
   if (__ballot(src >= 0) != 0) {
-    float bv[KS];
+    T bv[KS];
     if (L2L) {
-      const float* ps = in + (size_t)(src >= 0 ? src : 0) * parts * P2 + kq * KS;
+      const T* ps = in + (size_t)(src >= 0 ? src : 0) * parts * P2 + kq * KS;
 #pragma unroll
-      for (int ks = 0; ks < KS; ks++) bv[ks] = (src >= 0 && kq * KS + ks < P2) ? ps[ks] : 0.f;
+      for (int ks = 0; ks < KS; ks++) bv[ks] = (src >= 0 && kq * KS + ks < P2) ? ps[ks] : T(0);
     } else {
-      const float4* ms = reinterpret_cast<const float4*>(in + (size_t)(src >= 0 ? src : 0) * parts * ML::VS + kq * ML::KSP);
+      const V4* ms = reinterpret_cast<const V4*>(in + (size_t)(src >= 0 ? src : 0) * parts * ML::VS + kq * ML::KSP);
 #pragma unroll
       for (int v4 = 0; v4 < ML::KSP / 4; v4++) {
-        const float4 m4 = src >= 0 ? ms[v4] : make_float4(0.f, 0.f, 0.f, 0.f);
-        if (4 * v4 + 0 < KS) bv[4 * v4 + 0] = (kq * KS + 4 * v4 + 0 < P2) ? m4.x : 0.f;
-        if (4 * v4 + 1 < KS) bv[4 * v4 + 1] = (kq * KS + 4 * v4 + 1 < P2) ? m4.y : 0.f;
-        if (4 * v4 + 2 < KS) bv[4 * v4 + 2] = (kq * KS + 4 * v4 + 2 < P2) ? m4.z : 0.f;
-        if (4 * v4 + 3 < KS) bv[4 * v4 + 3] = (kq * KS + 4 * v4 + 3 < P2) ? m4.w : 0.f;
+        const V4 m4 = src >= 0 ? ms[v4] : V4{T(0), T(0), T(0), T(0)};
+        if (4 * v4 + 0 < KS) bv[4 * v4 + 0] = (kq * KS + 4 * v4 + 0 < P2) ? m4[0] : T(0);
+        if (4 * v4 + 1 < KS) bv[4 * v4 + 1] = (kq * KS + 4 * v4 + 1 < P2) ? m4[1] : T(0);
+        if (4 * v4 + 2 < KS) bv[4 * v4 + 2] = (kq * KS + 4 * v4 + 2 < P2) ? m4[2] : T(0);
+        if (4 * v4 + 3 < KS) bv[4 * v4 + 3] = (kq * KS + 4 * v4 + 3 < P2) ? m4[3] : T(0);
       }
     }
-    const float* A = opF + (size_t)oct * FR + l;
+    const T* A = opF + (size_t)oct * FR + l;
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) {
-      float af[MT];
+      T af[MT];
 #pragma unroll
       for (int mt = 0; mt < MT; mt++) af[mt] = A[(ks * MT + mt) * 64];
 #pragma unroll
-      for (int mt = 0; mt < MT; mt++) acc[mt] = Mfma<float>::fma(af[mt], bv[ks], acc[mt]);
+      for (int mt = 0; mt < MT; mt++) acc[mt] = Mfma<T>::fma(af[mt], bv[ks], acc[mt]);
     }
   }
   if (L2L) {
@@ -222,16 +226,16 @@ __global__ __launch_bounds__(L2L ? 256 : 512) void k_translate_mfma(int nout, co
     for (int mt = 0; mt < MT; mt++)
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        const int i = 16 * mt + 4 * kq + r;
+        const int i = 16 * mt + (D ? 4 * r + kq : 4 * kq + r);
         if (i < P2) {
-          float* o = out + (size_t)dst * parts * P2 + i;
+          T* o = out + (size_t)dst * parts * P2 + i;
           *o = add ? *o + acc[mt][r] : acc[mt][r];
         }
       }
     return;
   }
   // M2M: the 8 octant products through LDS, summed in octant order
-  __shared__ float red[8][MT * 4 * 64];
+  __shared__ T red[8][MT * 4 * 64];
 #pragma unroll
   for (int mt = 0; mt < MT; mt++)
 #pragma unroll
@@ -242,9 +246,10 @@ __global__ __launch_bounds__(L2L ? 256 : 512) void k_translate_mfma(int nout, co
     if (b >= nout) continue;
     // padded position -> slot (pads are written as zeros)
     const int seg = pos / ML::KSP, ks = pos % ML::KSP, i = seg * KS + ks;
-    float v = 0.f;
+    T v = T(0);
     if (ks < KS && i < P2) {
-      const int q = ((i >> 4) * 4 + (i & 3)) * 64 + ((i >> 2) & 3) * 16 + jb;
+      const int lo = i & 3, hi = (i >> 2) & 3;
+      const int q = ((i >> 4) * 4 + (D ? hi : lo)) * 64 + (D ? lo : hi) * 16 + jb;
 #pragma unroll
       for (int o = 0; o < 8; o++) v += red[o][q];
     }
@@ -257,16 +262,22 @@ __global__ __launch_bounds__(L2L ? 256 : 512) void k_translate_mfma(int nout, co
 int Engine::run_m2m(int lev) {
   const int nbp = sj.nb[lev];
   if (nbp == 0) return FMMX_OK;
-  if (!fp64) {
+  if (!fp64 || (!hh && p <= P_ALL)) {
     return dispatch_p(p, [&](auto pc) -> int {
       constexpr int P = decltype(pc)::value;
-      k_translate_mfma<P, 0><<<dim3((nbp + 15) / 16, parts()), 512, 0, stream>>>(
-          nbp, sj.cfirst[lev].as<int>(), sj.bkey[lev + 1].as<uint32_t>(), nullptr, nullptr, nullptr,
-          mexp[lev + 1].as<float>(), mexp[lev].as<float>(), m2m_ops<float>(lev), 0, parts());
+      auto go = [&](auto t) {
+        using T = typename decltype(t)::type;
+        k_translate_mfma<P, 0, T><<<dim3((nbp + 15) / 16, parts()), 512, 0, stream>>>(
+            nbp, sj.cfirst[lev].as<int>(), sj.bkey[lev + 1].as<uint32_t>(), nullptr, nullptr, nullptr,
+            mexp[lev + 1].as<T>(), mexp[lev].as<T>(), m2m_ops<T>(lev), 0, parts());
+      };
+      if (fp64) go(tag<double>{});
+      else go(tag<float>{});
       FMMX_HIP(hipGetLastError());
       return FMMX_OK;
     });
   }
+  // FP64 Helmholtz and the order above P_ALL: vector units
   const dim3 grid((nbp + TR_TB - 1) / TR_TB, 8);
   const long n = (long)nbp * VS * parts();
   int rc = m2m_part.ensure((size_t)8 * n * 8);
@@ -297,24 +308,29 @@ int Engine::run_m2m(int lev) {
     FMMX_HIP(hipGetLastError());
     return FMMX_OK;
   };
-  return p > P_ALL ? dispatch_hi(p, m2m) : dispatch_p(p, m2m);
+  return dispatch_hi(p, m2m);
 }
 
 int Engine::run_l2l(int lev, bool add) {
   const int nbc = si.nb[lev];
   if (nbc == 0) return FMMX_OK;
-  if (!fp64) {
+  if (!fp64 || (!hh && p <= P_ALL)) {
     // one wave per 16 children of a class: at most nbc / 16 + 8 waves
     return dispatch_p(p, [&](auto pc) -> int {
       constexpr int P = decltype(pc)::value;
-      k_translate_mfma<P, 1><<<dim3((nbc / 16 + 8 + 3) / 4, parts()), 256, 0, stream>>>(
-          nbc, nullptr, nullptr, si.parent[lev].as<int>(), cls_cnt[lev].as<int>(), cls_ord[lev].as<uint32_t>(),
-          lexp[lev - 1].as<float>(), lexp[lev].as<float>(), l2l_ops<float>(lev), add ? 1 : 0, parts());
+      auto go = [&](auto t) {
+        using T = typename decltype(t)::type;
+        k_translate_mfma<P, 1, T><<<dim3((nbc / 16 + 8 + 3) / 4, parts()), 256, 0, stream>>>(
+            nbc, nullptr, nullptr, si.parent[lev].as<int>(), cls_cnt[lev].as<int>(), cls_ord[lev].as<uint32_t>(),
+            lexp[lev - 1].as<T>(), lexp[lev].as<T>(), l2l_ops<T>(lev), add ? 1 : 0, parts());
+      };
+      if (fp64) go(tag<double>{});
+      else go(tag<float>{});
       FMMX_HIP(hipGetLastError());
       return FMMX_OK;
     });
   }
-  if (add) return fail(FMMX_ESTATE, "the L2L add form is FP32 only");
+  if (add) return fail(FMMX_ESTATE, "the L2L add form is on MFMA only");
   const int grid = (nbc + TR_TB - 1) / TR_TB + 8;
   if (hh) {
     return dispatch_hp(p, [&](auto pc) -> int {
@@ -334,7 +350,7 @@ int Engine::run_l2l(int lev, bool add) {
     FMMX_HIP(hipGetLastError());
     return FMMX_OK;
   };
-  return p > P_ALL ? dispatch_hi(p, l2l) : dispatch_p(p, l2l);
+  return dispatch_hi(p, l2l);
 }
 
 }  // namespace fmmx
