@@ -188,7 +188,7 @@ struct Engine {
   int graph_launch();
   // stand-alone Morton sort (fmmx_sort): staging, keys, permutation
   DevBuf srt_in[3], srt_keys_in, srt_idx_in, srt_keys, srt_perm, srt_bad;
-  DevBuf occ_bits;  // points per box of levels 8..0 and their statistics (automatic depth)
+  DevBuf occ_bits;  // points per level-8 cell and the box statistics (automatic depth)
   // box statistics the last automatic depth was chosen from
   long occ_boxes[MAXL + 1] = {};
   double occ_sumsq[MAXL + 1] = {};
@@ -220,6 +220,7 @@ struct Engine {
 
   DevBuf op_m2l_of;       // FP64 orbit operators (op_m2l is not uploaded with them)
   bool orb64_ok = false;
+  bool occ_clean = false;  // the counts of occ_bits are zero
   ~Engine();
   int init(const fmmx_config* c, int dev, void* stream);
   int set_points(int ni, const float* xi, const float* yi, const float* zi, const float* nxi, const float* nyi,

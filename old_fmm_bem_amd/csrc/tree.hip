@@ -595,7 +595,8 @@ __global__ __launch_bounds__(CL_T) void k_class_place(ClassLevels L) {
 // ---------------------------------------------------------------------
 // Box statistics of every level (automatic depth): the points per level-8
 // cell, counted in Morton order so that the 8 children of a box are 8
-// consecutive counts; each level's counts are the sums of its children's.
+// consecutive counts (and a flag per level-5 box that holds a point); each
+// level's counts are the sums of its children's.
 // Per level l: boxes[l] = boxes holding a point, sumsq[l] = sum of the
 // squared counts (the near-field pair count of a box grows with it).
 constexpr int OCC_L = 8;
@@ -603,7 +604,7 @@ constexpr long OCC_CELLS = 1L << (3 * OCC_L);  // 2^24 counts, 64 MB
 
 __global__ void k_occ_mark(int n, const float* __restrict__ x, const float* __restrict__ y,
                            const float* __restrict__ z, float xmin, float ymin, float zmin, double rbinv,
-                           unsigned* __restrict__ cnt) {
+                           unsigned* __restrict__ cnt, unsigned* __restrict__ flag) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   uint32_t k = 0xffffffffu;
   if (i < n) {
@@ -619,42 +620,116 @@ __global__ void k_occ_mark(int n, const float* __restrict__ x, const float* __re
   const unsigned long long same = __ballot(k == k0 && i < n);
   const unsigned long long act = __ballot(i < n);
   if (same == act) {
-    if ((threadIdx.x & 63) == 0 && act) atomicAdd(&cnt[k0], (unsigned)__popcll(act));
+    if ((threadIdx.x & 63) == 0 && act) {
+      atomicAdd(&cnt[k0], (unsigned)__popcll(act));
+      flag[k0 >> 9] = 1u;
+    }
   } else if (i < n) {
     atomicAdd(&cnt[k], 1u);
+    flag[k >> 9] = 1u;
   }
 }
 
-// one level up: out[b] = sum of in[8b .. 8b+7] for nout boxes, and the
-// statistics of the input level, st[0] += occupied boxes, st[1] += sum of
-// squared counts (one atomic pair per workgroup)
-__global__ __launch_bounds__(256) void k_occ_up(long nout, const unsigned* __restrict__ in,
-                                                unsigned* __restrict__ out, unsigned long long* __restrict__ st) {
-  __shared__ unsigned long long red[2][4];
-  unsigned long long nb = 0, sq = 0;
-  for (long b = (long)blockIdx.x * 256 + threadIdx.x; b < nout; b += (long)gridDim.x * 256) {
-    const uint4 a = *(const uint4*)(in + 8 * b), c = *(const uint4*)(in + 8 * b + 4);
-    const unsigned v[8] = {a.x, a.y, a.z, a.w, c.x, c.y, c.z, c.w};
-    unsigned t = 0;
-    for (int k = 0; k < 8; k++) {
-      t += v[k];
-      nb += v[k] != 0;
-      sq += (unsigned long long)v[k] * v[k];
+// Statistics of levels 8..5 and the counts of the level-4 boxes, in one pass
+// that leaves counts and flags cleared for the next call.  A workgroup takes
+// OCC_B4 level-4 boxes of 4,096 cells, 16 consecutive cells per thread: 2 boxes
+// of level 7 per thread, one of level 6 per 4 lanes, one of level 5 per 32, which
+// are skipped where no point set their flag.  part: the workgroup's sums
+// (boxes, sum of squares of levels 8, 7, 6, 5).  Bound by the 64 MB read where
+// all cells' boxes hold points; a fill and eight launches, one per level, took
+// 83 us of 250,000 points in a cube, 70 us of 1,000; this and k_occ_top 26 and 16.
+constexpr int OCC_B4 = 8, OCC_WG = 4096 / OCC_B4;
+static_assert(OCC_L == 8, "levels 8..5 of a 4,096-cell box, 4..1 in k_occ_top");
+__global__ __launch_bounds__(256) void k_occ_cells(unsigned* __restrict__ cnt, unsigned* __restrict__ flag,
+                                                   unsigned* __restrict__ lvl4,
+                                                   unsigned long long* __restrict__ part) {
+  __shared__ unsigned w4[OCC_B4][4];
+  __shared__ unsigned long long red[4][8];
+  const int tid = threadIdx.x, lane = tid & 63;
+  unsigned long long st[8] = {};
+  auto count = [&](int k, unsigned v) {
+    st[k] += v != 0;
+    st[k + 1] += (unsigned long long)v * v;
+  };
+  for (int k = 0; k < OCC_B4; k++) {
+    const size_t b4 = (size_t)blockIdx.x * OCC_B4 + k;
+    unsigned* f = flag + b4 * 8 + (tid >> 5);
+    unsigned s = 0;
+    if (*f) {
+      uint4* c = reinterpret_cast<uint4*>(cnt + b4 * 4096 + tid * 16);
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        const uint4 u = c[2 * h], v = c[2 * h + 1];
+        const unsigned a[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+        unsigned t = 0;
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+          t += a[q];
+          count(0, a[q]);
+        }
+        count(2, t);
+        s += t;
+        if (u.x | u.y | u.z | u.w) c[2 * h] = make_uint4(0, 0, 0, 0);
+        if (v.x | v.y | v.z | v.w) c[2 * h + 1] = make_uint4(0, 0, 0, 0);
+      }
+      if ((tid & 31) == 0) *f = 0;
     }
-    out[b] = t;
+    s += __shfl_xor(s, 1);
+    s += __shfl_xor(s, 2);
+    if ((lane & 3) == 0) count(4, s);
+    for (int o = 4; o < 32; o <<= 1) s += __shfl_xor(s, o);
+    if ((lane & 31) == 0) count(6, s);
+    s += __shfl_xor(s, 32);
+    if (lane == 0) w4[k][tid >> 6] = s;
   }
-  for (int o = 32; o > 0; o >>= 1) {
-    nb += __shfl_xor(nb, o);
-    sq += __shfl_xor(sq, o);
-  }
-  if ((threadIdx.x & 63) == 0) {
-    red[0][threadIdx.x >> 6] = nb;
-    red[1][threadIdx.x >> 6] = sq;
+#pragma unroll
+  for (int q = 0; q < 8; q++) {
+    for (int o = 32; o > 0; o >>= 1) st[q] += __shfl_xor(st[q], o);
+    if (lane == 0) red[tid >> 6][q] = st[q];
   }
   __syncthreads();
-  if (threadIdx.x < 2) {
-    const unsigned long long v = red[threadIdx.x][0] + red[threadIdx.x][1] + red[threadIdx.x][2] + red[threadIdx.x][3];
-    if (v) atomicAdd(&st[threadIdx.x], v);
+  if (tid < OCC_B4) lvl4[blockIdx.x * OCC_B4 + tid] = w4[tid][0] + w4[tid][1] + w4[tid][2] + w4[tid][3];
+  if (tid < 8) part[blockIdx.x * 8 + tid] = red[0][tid] + red[1][tid] + red[2][tid] + red[3][tid];
+}
+
+// levels 4..1 (thread: a level-3 box, wave: a level-1 box) and the workgroups'
+// sums of the levels below; st[2 l], st[2 l + 1]: boxes and sum of squares
+__global__ __launch_bounds__(512) void k_occ_top(const unsigned* __restrict__ lvl4,
+                                                 const unsigned long long* __restrict__ part,
+                                                 unsigned long long* __restrict__ out) {
+  static_assert(OCC_WG == 512, "one workgroup of k_occ_cells per thread");
+  __shared__ unsigned long long red[8][16];
+  const int tid = threadIdx.x, lane = tid & 63;
+  unsigned long long st[16] = {};  // levels 8..1
+  auto count = [&](int k, unsigned v) {
+    st[k] += v != 0;
+    st[k + 1] += (unsigned long long)v * v;
+  };
+#pragma unroll
+  for (int q = 0; q < 8; q++) st[q] = part[tid * 8 + q];
+  const uint4 u = reinterpret_cast<const uint4*>(lvl4)[2 * tid], v = reinterpret_cast<const uint4*>(lvl4)[2 * tid + 1];
+  const unsigned a[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+  unsigned s = 0;
+#pragma unroll
+  for (int q = 0; q < 8; q++) {
+    s += a[q];
+    count(8, a[q]);
+  }
+  count(10, s);
+  for (int o = 1; o < 8; o <<= 1) s += __shfl_xor(s, o);
+  if ((lane & 7) == 0) count(12, s);
+  for (int o = 8; o < 64; o <<= 1) s += __shfl_xor(s, o);
+  if (lane == 0) count(14, s);
+#pragma unroll
+  for (int q = 0; q < 16; q++) {
+    for (int o = 32; o > 0; o >>= 1) st[q] += __shfl_xor(st[q], o);
+    if (lane == 0) red[tid >> 6][q] = st[q];
+  }
+  __syncthreads();
+  if (tid < 16) {
+    unsigned long long t = 0;
+    for (int w = 0; w < 8; w++) t += red[w][tid];
+    out[2 * (OCC_L - tid / 2) + (tid & 1)] = t;
   }
 }
 
@@ -979,33 +1054,25 @@ int Engine::occupancy(int n, const float* x, const float* y, const float* z, lon
   if (n <= 0) return FMMX_OK;
   static_assert(OCC_L == MAXL, "statistics from the deepest level");
   int rc;
-  // counts of levels 8..0 (level l: 8^l words) then 2 words of statistics
-  // per level
-  long words = 0;
-  for (int l = 0; l <= OCC_L; l++) words += 1L << (3 * l);
-  const long st_off = (words + 3) / 4 * 4;  // 16-byte aligned
-  if ((rc = occ_bits.ensure((size_t)(st_off + 4 * (OCC_L + 1)) * 4))) return rc;
+  // level-8 counts and level-5 flags, zero between calls; then level-4 counts,
+  // the workgroups' sums and 2 words of statistics per level (8-byte each)
+  const size_t flags = OCC_CELLS, lvl4 = flags + (1 << 15), part = lvl4 + 4096, st_off = part + OCC_WG * 16;
+  const size_t had = occ_bits.bytes;
+  if ((rc = occ_bits.ensure((st_off + 4 * (OCC_L + 1)) * 4))) return rc;
   unsigned* base = occ_bits.as<unsigned>();
-  unsigned* lvl[OCC_L + 1];
-  long o = 0;
-  for (int l = OCC_L; l >= 0; l--) {
-    lvl[l] = base + o;  // level l starts at a multiple of 8 words (16-byte aligned for l >= 1)
-    o += 1L << (3 * l);
-  }
   unsigned long long* st = (unsigned long long*)(base + st_off);
-  k_fill_int<<<(int)((st_off + 4 * (OCC_L + 1) + TPB - 1) / TPB), TPB, 0, stream>>>(st_off + 4 * (OCC_L + 1), 0,
-                                                                                    (int*)base);
+  if (occ_bits.bytes != had || !occ_clean)
+    k_fill_int<<<(int)((lvl4 + TPB - 1) / TPB), TPB, 0, stream>>>((long)lvl4, 0, (int*)base);
+  occ_clean = false;
   const double rbinv = (double)((float)(1 << OCC_L) / rd);
-  k_occ_mark<<<nblk(n), TPB, 0, stream>>>(n, x, y, z, xmin, ymin, zmin, rbinv, lvl[OCC_L]);
-  for (int l = OCC_L; l >= 1; l--) {
-    const long nout = 1L << (3 * (l - 1));
-    const int g = (int)std::min<long>(1024, (nout + 255) / 256);
-    k_occ_up<<<g, 256, 0, stream>>>(nout, lvl[l], lvl[l - 1], st + 2 * l);
-  }
+  k_occ_mark<<<nblk(n), TPB, 0, stream>>>(n, x, y, z, xmin, ymin, zmin, rbinv, base, base + flags);
+  k_occ_cells<<<OCC_WG, 256, 0, stream>>>(base, base + flags, base + lvl4, (unsigned long long*)(base + part));
+  k_occ_top<<<1, 512, 0, stream>>>(base + lvl4, (const unsigned long long*)(base + part), st);
   if (!rb_host) FMMX_HIP(hipHostMalloc((void**)&rb_host, RB_INTS * 4, hipHostMallocDefault));
   static_assert(4 * (MAXL + 1) <= RB_INTS, "readback buffer");
   FMMX_HIP(hipMemcpyAsync(rb_host, st, (size_t)2 * (OCC_L + 1) * 8, hipMemcpyDeviceToHost, stream));
   FMMX_HIP(hipStreamSynchronize(stream));
+  occ_clean = true;
   const unsigned long long* h = (const unsigned long long*)rb_host;
   boxes[0] = 1;
   sumsq[0] = (double)n * (double)n;
