@@ -12,9 +12,11 @@ namespace {
 //   YK 1: Yukawa multipoles, M~_n^m = sum q i~_n(lambda rho)/i~_n(lambda rb)
 //       (rho/rb)^n conj(Y_n^m): the Laplace harmonics times a radial weight
 //       per degree (lrb = lambda rb)
-//   YK 2: Helmholtz multipoles of one part of the charges (real or
-//       imaginary), M_n^m = sum q j^_n(k rho) (rho/rb)^n conj(Y_n^m)
-//       (lrb = k rb)
+//   YK 2: Helmholtz multipoles, M_n^m = sum q j^_n(k rho) (rho/rb)^n
+//       conj(Y_n^m) (lrb = k rb), of the real charges q and the imaginary ones
+//       q2 (VS behind).  Both parts in one pass: the Bessel series in FP64 and
+//       the harmonics are most of the work (sphere of 1M points, p = 12, beside the near
+//       field: 0.96 ms as a pass per part, 0.86 ms here)
 //   Box b's multipole starts at M + b * mstride + moff.
 template <int P, typename T, int YK = 0, int HALF = 0, int CONV = -1, int GN = -1>
 __global__ __launch_bounds__(64) void k_p2m(int nb, const uint32_t* __restrict__ bkey, const int* __restrict__ bfirst,
@@ -24,11 +26,11 @@ __global__ __launch_bounds__(64) void k_p2m(int nb, const uint32_t* __restrict__
                                             const float* __restrict__ nz, const float* __restrict__ q, int gn,
                                             int conv, int lev, double xmin, double ymin, double zmin, double rb,
                                             const double* __restrict__ corr, T* __restrict__ M, double lrb,
-                                            int mstride, int moff) {
+                                            int mstride, int moff, const float* __restrict__ q2) {
   // HALF: two leaves per wave, rows 0-31 for the first and 32-63 for the
   // second, for leaves of at most about 32 particles
   constexpr int NR = P * (P + 1) / 2, P2 = P * P, NL = HALF ? 2 : 1, STEP = 64 / NL;
-  constexpr int NC = (NL * P2 + 63) / 64;
+  constexpr int NC = (NL * P2 + 63) / 64, PARTS = YK == 2 ? 2 : 1;
   __shared__ T red[64][P2 + 1];
   const int lane = threadIdx.x, h = HALF ? lane >> 5 : 0, sub = HALF ? lane & 31 : lane;
   const int b = HALF ? 2 * (int)blockIdx.x + h : (int)blockIdx.x;
@@ -37,14 +39,53 @@ __global__ __launch_bounds__(64) void k_p2m(int nb, const uint32_t* __restrict__
   double cx = 0, cy = 0, cz = 0;
   if (valid) box_center(bkey[b], lev, xmin, ymin, zmin, rb, cx, cy, cz);
   const double rbinv = 1.0 / rb;
-  T acc[NC];
+  T acc[PARTS][NC];
 #pragma unroll
-  for (int c = 0; c < NC; c++) acc[c] = T(0);
+  for (int t = 0; t < PARTS; t++)
+#pragma unroll
+    for (int c = 0; c < NC; c++) acc[t][c] = T(0);
+  // column sums: entry idx = (leaf of the wave, column) over that leaf's rows
+  auto sums = [&](int t) __attribute__((always_inline)) {
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+      const int idx = lane + 64 * c, hh = idx / P2, col = idx % P2;
+      if (hh < NL) {
+        T s = T(0);
+        for (int r = 0; r < STEP; r++) s += red[hh * STEP + r][col];
+        acc[t][c] += s;
+      }
+    }
+    __syncthreads();
+  };
   const int i0 = valid ? bfirst[b] : 0, i1 = valid ? blast[b] : -1;
   for (int base = 0;; base += STEP) {
     if (__ballot(i0 + base <= i1) == 0) break;  // one wave per block: uniform
     const int i = i0 + base + sub;
     T* row = red[lane];
+    if constexpr (YK == 2) {
+      double ux = 0, uy = 0, uz = 0, jx[P];
+      if (i <= i1)
+        eff_point(CONV >= 0 ? CONV : conv, (double)x[i] - cx, (double)y[i] - cy, (double)z[i] - cz, rbinv, ux, uy, uz);
+      T Sr[NR], Si[NR];
+      solid_harmonics<P, T>(T(ux), T(uy), T(uz), Sr, Si);
+      jhat_dev<P - 1>(lrb * sqrt(ux * ux + uy * uy + uz * uz), jx);
+#pragma unroll
+      for (int t = 0; t < PARTS; t++) {
+        const double qd = i <= i1 ? (double)(t ? q2 : q)[i] : 0.0;
+#pragma unroll
+        for (int n = 0; n < P; n++) {
+          const T w = T(qd * jx[n]);
+#pragma unroll
+          for (int m = 0; m <= n; m++) {
+            row[sl(n, m)] = w * Sr[sl(n, m)];
+            if (m > 0) row[NR + n * (n - 1) / 2 + m - 1] = -w * Si[sl(n, m)];
+          }
+        }
+        sums(t);
+      }
+      continue;
+    }
     if (YK == 0 && CONV == FMMX_CONV_EXACT && GN == 0 && i <= i1) {
       // charges in the EXACT convention (unit table ratios): the harmonics
       // column by column straight into the LDS row; the unrolled recurrence
@@ -92,16 +133,12 @@ __global__ __launch_bounds__(64) void k_p2m(int nb, const uint32_t* __restrict__
       if (YK) {
         double ib0[P], ibx[P];
         const double lr = lrb * sqrt(ux * ux + uy * uy + uz * uz);
-        if (YK == 2) {
-          jhat_dev<P - 1>(lr, ibx);
-        } else {
-          ibar_dev<P - 1>(lrb, ib0);
-          ibar_dev<P - 1>(lr, ibx);
-        }
+        ibar_dev<P - 1>(lrb, ib0);
+        ibar_dev<P - 1>(lr, ibx);
         const double qd = (double)q[i];
 #pragma unroll
         for (int n = 0; n < P; n++) {
-          const T w = T(YK == 2 ? qd * ibx[n] : qd * ibx[n] / ib0[n]);
+          const T w = T(qd * ibx[n] / ib0[n]);
 #pragma unroll
           for (int m = 0; m <= n; m++) {
             row[sl(n, m)] = w * Sr[sl(n, m)];
@@ -140,31 +177,23 @@ __global__ __launch_bounds__(64) void k_p2m(int nb, const uint32_t* __restrict__
 #pragma unroll
       for (int c = 0; c < P2; c++) row[c] = T(0);
     }
-    __syncthreads();
-    // column sums: entry idx = (leaf of the wave, column) over that leaf's rows
-#pragma unroll
-    for (int c = 0; c < NC; c++) {
-      const int idx = lane + 64 * c, hh = idx / P2, col = idx % P2;
-      if (hh < NL) {
-        T s = T(0);
-        for (int r = 0; r < STEP; r++) s += red[hh * STEP + r][col];
-        acc[c] += s;
-      }
-    }
-    __syncthreads();
+    sums(0);
   }
   using ML = MLayout<P>;
   const int b0 = HALF ? 2 * (int)blockIdx.x : (int)blockIdx.x;
 #pragma unroll
-  for (int c = 0; c < NC; c++) {
-    const int idx = lane + 64 * c, hh = idx / P2, col = idx % P2;
-    if (hh < NL && b0 + hh < nb) M[(size_t)(b0 + hh) * mstride + moff + ML::at(col)] = acc[c];
-  }
+  for (int t = 0; t < PARTS; t++)
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+      const int idx = lane + 64 * c, hh = idx / P2, col = idx % P2;
+      if (hh < NL && b0 + hh < nb) M[(size_t)(b0 + hh) * mstride + moff + t * ML::VS + ML::at(col)] = acc[t][c];
+    }
   // zero the padding slots (M2M applies its operator to whole stored vectors)
   for (int c2 = lane; c2 < NL * ML::VS; c2 += 64) {
     const int hh = c2 / ML::VS, c = c2 % ML::VS;
     if (b0 + hh < nb && (c % ML::KSP >= ML::KS || (c / ML::KSP) * ML::KS + c % ML::KSP >= P2))
-      M[(size_t)(b0 + hh) * mstride + moff + c] = T(0);
+#pragma unroll
+      for (int t = 0; t < PARTS; t++) M[(size_t)(b0 + hh) * mstride + moff + t * ML::VS + c] = T(0);
   }
 }
 
@@ -389,7 +418,7 @@ int Engine::run_p2m(int neq) {
       nb, sj.bkey[lmax].as<uint32_t>(), sj.bfirst[lmax].as<int>(), sj.blast.as<int>(), sj.x.as<float>(),         \
       sj.y.as<float>(), sj.z.as<float>(), sj.nx.as<float>(), sj.ny.as<float>(), sj.nz.as<float>(), Q_,            \
       neq == FMMX_GNJ, cfg.convention, lmax, xmin, ymin, zmin, rb(lmax), corr, mexp[lmax].as<T_>(), lrb, STRIDE_, \
-      OFF_)
+      OFF_, qs2.as<float>())
     // Laplace charges in the EXACT convention: the streaming form
 #define FMMX_P2M_H(T_, YK_, H_, Q_, STRIDE_, OFF_)                                                 \
   do {                                                                                            \
@@ -417,10 +446,8 @@ int Engine::run_p2m(int neq) {
       if constexpr (P % 2 == 0 && P >= 4) {
         if (fp64) {
           FMMX_P2M(double, 2, qs.as<float>(), 2 * VS, 0);
-          FMMX_P2M(double, 2, qs2.as<float>(), 2 * VS, VS);
         } else {
           FMMX_P2M(float, 2, qs.as<float>(), 2 * VS, 0);
-          FMMX_P2M(float, 2, qs2.as<float>(), 2 * VS, VS);
         }
       } else {
         return fail(FMMX_EUNSUPPORTED, "Helmholtz needs p in {4, 6, 8, 10, 12}");
