@@ -49,12 +49,14 @@ def parse():
     return ap.parse_args()
 
 
-def traffic_from_profile(n, p, lmax, all_levels, split):
+def traffic_from_profile(n, p, lmax, all_levels, split, orbit):
     """HBM bytes per M2L launch (every level in one launch, or the leaf
     level's) measured with rocprofv3 PMC counters (FETCH_SIZE + WRITE_SIZE,
     scaled by a plain copy of known size), kept as a text summary under
     profiles/; None when no summary matches this workload."""
-    if split:
+    if orbit:
+        name = "k_m2l_orbit_all_levels_n1m_p10_pmc.txt"
+    elif split:
         name = "k_m2l_split_all_levels_n1m_p10_pmc.txt"
     else:
         name = "k_m2l_all_levels_n1m_p10_pmc.txt" if all_levels else "k_m2l_leaf_n1m_p10_pmc.txt"
@@ -307,12 +309,17 @@ def main():
         e64 = float(torch.linalg.norm(v64[torch.from_numpy(idx).cuda()] - dv) / torch.linalg.norm(dv))
         fp64 = {"ms_per_step": ms64, "value": a.n / (ms64 * 1e3), "ms_eval_only": ms64_eval, "err_v": e64,
                 "phases_ms": {k: round(v_, 4) for k, v_ in ph64.items()}}
-        # the ratio's denominator against its own roof: the FP64 leaf M2L
-        # (vector FMA) on the FP64 peak
-        fl64 = 2.0 * a.p ** 4 * st64["m2l_pairs_leaf"]
+        # the ratio's denominator against its own roof: the FP64 M2L
+        # (one launch of all levels by reflection orbits, FP64 MFMA, for the
+        # orders that has; else the leaf level on vector FMA) on the FP64 peak
+        # (matrix = vector)
+        all64 = bool(st64["m2l_all_levels"])
+        fl64 = 2.0 * a.p ** 4 * st64["m2l_pairs" if all64 else "m2l_pairs_leaf"]
         ach64 = fl64 / (ph64["ms_m2l_leaf"] * 1e-3) / 1e12
-        fp64["roofline"] = {"bound": "valu", "achieved": ach64, "peak": PEAK["fp64_vector"], "unit": "TFLOP/s",
-                            "frac": ach64 / PEAK["fp64_vector"], "kernel": f"k_m2l_vec<{a.p}, double>, leaf level",
+        fp64["roofline"] = {"bound": "mfma" if all64 else "valu", "achieved": ach64, "peak": PEAK["fp64_vector"], "unit": "TFLOP/s",
+                            "frac": ach64 / PEAK["fp64_vector"],
+                            "kernel": f"k_m2l_of<{a.p}>, levels 2-{lmax} in one launch" if all64
+                            else f"k_m2l_vec<{a.p}, double>, leaf level",
                             "ms_per_launch": ph64["ms_m2l_leaf"]}
         f64.close()
 
@@ -324,14 +331,27 @@ def main():
     # engine's M2L runs on the FP16 matrix cores (error-compensated split:
     # three FP16 products per FP32-accurate product) or on FP32 MFMA.
     p2 = a.p * a.p
-    split = f.tuning[lmax][1] >= 3
+    split, orbit = f.tuning[lmax][1] >= 3, f.tuning[lmax][1] == 6
     launch_pairs = st["m2l_pairs"] if st["m2l_all_levels"] else st["m2l_pairs_leaf"]
     peak_m2l = PEAK["fp16_mfma"] if split else PEAK["fp32_mfma"]
     if phases["ms_m2l"] >= phases["ms_p2p"]:
         flops = 2.0 * p2 * p2 * launch_pairs
         achieved = flops / (phases["ms_m2l_leaf"] * 1e-3) / 1e12
-        tr = traffic_from_profile(a.n, a.p, lmax, st["m2l_all_levels"], split)
-        if split and f.tuning[lmax][1] == 5:
+        tr = traffic_from_profile(a.n, a.p, lmax, st["m2l_all_levels"], split, orbit)
+        if orbit:
+            # executed MFMA work per pair: 63 products for 189 pairs, each 8 tiles of 16 rows by
+            # 32-deep steps, three per octet of slots of a reflection class and two for the rest
+            size = [0] * 8
+            for n in range(a.p):
+                for m in range(n + 1):
+                    for im in range(2 if m else 1):
+                        size[((m ^ im) & 1) | im << 1 | ((n + m) & 1) << 2] += 1
+            no = 0
+            while sum(c > 4 * no for c in size) > 4 or max(size) > 4 * no + 4:
+                no += 1
+            executed = 63 / 189 * 2.0 * 128 * 32 * (3 * no + 2 * (max(size) > 4 * no))
+            kern = f"k_m2l_o (reflection orbits, FP16 split, v_mfma_f32_16x16x32_f16), levels 2-{lmax} in one launch"
+        elif split and f.tuning[lmax][1] == 5:
             # executed MFMA work per pair: 32 MT rows x 16 KH k-positions per target
             mt, ks = (p2 + 31) // 32, (p2 + 1) // 2
             kh = (3 * (ks + (ks & 1)) + 7) // 8

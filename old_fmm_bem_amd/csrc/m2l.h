@@ -1,6 +1,6 @@
 // m2l.h -- expansion layouts, reflection signs and launch descriptors shared
 // by the M2L kernels (m2l.hip: FP32 and FP64 forms; m2l_split.hip: the
-// error-compensated FP16 form).
+// error-compensated FP16 form; m2l_orbit*.hip: the reflection orbits).
 #pragma once
 
 #include "engine.h"

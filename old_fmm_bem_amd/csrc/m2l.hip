@@ -1,8 +1,9 @@
 // m2l.hip -- M2L (kernel/m2l.cxx) for CDNA4 (gfx950): targets of one parity
 // class share the same 189 lattice offsets, so a tile of targets runs as 189
 // GEMMs (operator [p^2 x p^2] x gathered source multipoles [p^2 x tile]); FP32
-// on MFMA, every level in one launch.  The launchers of the FP16 forms
-// (m2l_split.hip, m2l_orbit.hip) are here too.
+// on MFMA, every level in one launch.  The launchers of the FP16 and
+// orbit forms (m2l_split.hip, m2l_orbit.hip, m2l_orbit_gen.hip,
+// m2l_orbit_fp64.hip) are here too.
 #include "phases.h"
 
 namespace fmmx {

@@ -1,5 +1,5 @@
 // orbit.h -- device helpers of the reflection-orbit M2L kernels (m2l_orbit.hip,
-// m2l_orbit_gen.hip).
+// m2l_orbit_gen.hip, m2l_orbit_fp64.hip).
 #pragma once
 
 #include <type_traits>

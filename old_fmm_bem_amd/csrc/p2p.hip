@@ -1,6 +1,6 @@
 // p2p.hip -- near field and direct sums for CDNA4 (gfx950), wave64.
-//   P2P  kernel/G_p2p.cxx, Gni_p2p.cxx, Gnj_p2p.cxx: one workgroup per target
-//        leaf box (two lanes per target for small leaves), source particles
+//   P2P  kernel/G_p2p.cxx, Gni_p2p.cxx, Gnj_p2p.cxx: work items of a target
+//        leaf box (two or more lanes per target for small leaves), source particles
 //        of the near boxes staged through LDS, FP32 (or FP64) pair math, FP64
 //        per-target sums.
 //   direct sums kernel/G_dir.cxx, Gni_dir.cxx, Gnj_dir.cxx.
@@ -18,7 +18,7 @@ __device__ __forceinline__ float yexp(float x) { return __expf(x); }
 __device__ __forceinline__ double yexp(double x) { return exp(x); }
 
 // ---------------------------------------------------------------------
-// P2P: one workgroup per target leaf box (chunks of BS targets), sources of
+// P2P: a workgroup per work item (up to BS targets of a leaf box), sources of
 // each near box staged through LDS in tiles of BS.
 //
 // A staged source: in doubles where the pair computes in them (FP64, EXACT), so

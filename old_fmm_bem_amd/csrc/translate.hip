@@ -1,6 +1,6 @@
 // translate.hip -- M2M and L2L (kernel/m2m.cxx, l2l.cxx) for CDNA4 (gfx950):
 // dense p^2 x p^2 operators per child octant (level independent in the scaled
-// basis), on MFMA in FP32.
+// basis), on MFMA in FP32 and, but for Helmholtz and order 18, in FP64.
 #include "phases.h"
 
 namespace fmmx {
