@@ -757,7 +757,7 @@ int Engine::upload_operators() {
     if ((rc = upload<float>(op_m2m, S->m2m_frag, stream)) || (rc = upload<float>(op_l2l, S->l2l_frag, stream)) ||
         (rc = upload<float>(op_m2l, canon ? S->m2l_canon : S->m2l_frag, stream)))
       return rc;
-    // the FP16 forms' operators go up with their first launch (upload_split)
+    // the operators of the FP16 form in use go up behind the tree (upload_split)
     split_ok = canon && !S->m2l_split.empty();
     wide_ok = split_ok && !S->m2l_wide.empty();
     orb_ok = split_ok && !S->m2l_orbit.empty();
@@ -915,6 +915,12 @@ int Engine::set_points(int ni, const float* xi, const float* yi, const float* zi
   tree_stats_pending = true;
   have_points = true;
   last_neq = -1;
+  // the M2L operators of the form that an evaluation will take, once; a handle
+  // set up for Yukawa or Helmholtz gets them if it evaluates Laplace after all
+  if (split_ok && !(lam > 0) && !(hk > 0)) {
+    const int form = m2l_variant(lmax).pa;
+    if (form >= 3 && (rc = upload_split(form))) return rc;
+  }
   return FMMX_OK;
 }
 

@@ -128,7 +128,7 @@ struct Engine {
   DevBuf op_m2l_o, orbtab;
   bool orb_ok = false;
   bool orbit_fits() const;
-  // the operators of an FP16 M2L form on the device (at its first use)
+  // the operators of an FP16 M2L form on the device (once; set_points, or its first use)
   int upload_split(int form);
   bool up_h = false, up_w = false, up_o = false;
   bool m2l_split(int lev) const;  // the level's M2L runs the FP16 split kernel
