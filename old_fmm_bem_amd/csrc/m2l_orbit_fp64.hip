@@ -188,14 +188,11 @@ __global__ __launch_bounds__(F64_NTH) __attribute__((amdgpu_waves_per_eu(2, 2)))
 #pragma unroll
     for (int s = 0; s < 4; s++) hand[s] = v[s];
   };
-  // n fragments of a step into LDS buffer b, without registers (k_m2l_og)
+  // n fragments of a step into LDS buffer b; sync() waits for them
   auto copy = [&](const u32x4* from, int b, int n) __attribute__((always_inline)) {
 #pragma unroll
     for (int e = 0; e < CH; e += F64_NTH)
-      if (e + w * 64 < n)
-        asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(as_base + (b * CH + e + w * 64) * 16),
-                     "v"(from + e + tid)
-                     : "memory", "m0");
+      if (e + w * 64 < n) lds_copy16(as_base + (b * CH + e + w * 64) * 16, from + e + tid);
   };
   auto op_src = [&](int o) __attribute__((always_inline)) -> const u32x4* { return opH + (size_t)(otab[o].w & 0xff) * F::FRO; };
   // every access of the step behind has arrived in every wave

@@ -233,15 +233,10 @@ __global__ __launch_bounds__(GEN_NTH) __attribute__((amdgpu_waves_per_eu(2, 2)))
 #pragma unroll
     for (int s = 0; s < 4; s++) hand[s][0] = v[s][0], hand[s][1] = v[s][1];
   };
-  // a step's fragments into LDS buffer b, without registers.  Written out so
-  // that the compiler does not hold every LDS read behind it back until the
-  // copies have landed; sync() waits for them.
+  // a step's fragments into LDS buffer b; sync() waits for them
   auto copy = [&](const u32x4* from, int b) __attribute__((always_inline)) {
 #pragma unroll
-    for (int e = 0; e < CH; e += GEN_NTH)
-      asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(as_base + (b * CH + e + w * 64) * 16),
-                   "v"(from + e + tid)
-                   : "memory", "m0");
+    for (int e = 0; e < CH; e += GEN_NTH) lds_copy16(as_base + (b * CH + e + w * 64) * 16, from + e + tid);
   };
   auto op_src = [&](int o) __attribute__((always_inline)) -> const u32x4* { return opH + (size_t)(otab[o].w & 0xff) * FRO; };
   // every access of the step behind has arrived in every wave

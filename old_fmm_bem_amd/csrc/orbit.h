@@ -63,6 +63,15 @@ __device__ __forceinline__ uint32_t lo_pair(float a, float b, uint32_t h) {
   return hi_pair(ra, rb);
 }
 
+// 16 bytes per lane from global memory to LDS, the wave's 1,024 bytes at dst,
+// without registers.  Written out so that the compiler does not hold every LDS
+// read behind it back until the copy has landed; the caller waits for it.  The
+// scalar write of M0 and the copy that reads it need a wait state between them,
+// which the compiler puts into its own code but not into this.
+__device__ __forceinline__ void lds_copy16(uint32_t dst, const u32x4* from) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(dst), "v"(from) : "memory", "m0");
+}
+
 }  // namespace
 
 }  // namespace fmmx
