@@ -1029,10 +1029,21 @@ int Engine::evaluate(int neq, const float* qj, double* vi, double* gxi, double* 
   // Without per-phase timing the near field (vector ALU) runs on the second
   // stream beside the far field (MFMA); L2P, which adds to its results, waits.
   const bool overlap = overlap_on && !per_phase && aux && ni > 0;
+  // the side streams join the caller's on every way out: after an error, too, its
+  // next call may rebuild what their launches still read
+  struct Join {
+    hipStream_t main, side[2] = {};
+    hipEvent_t done[2];
+    ~Join() {
+      for (int k = 0; k < 2; k++)
+        if (side[k] && hipEventRecord(done[k], side[k]) == hipSuccess) (void)hipStreamWaitEvent(main, done[k], 0);
+    }
+  } join{stream, {}, {ev[11], ev[13]}};
   if (ni > 0) {
     if (overlap) {
       FMMX_HIP(hipEventRecord(ev[10], stream));
       FMMX_HIP(hipStreamWaitEvent(aux, ev[10], 0));
+      join.side[0] = aux;
       hipStream_t main = stream;
       stream = aux;
       rc = run_p2p(neq);
@@ -1057,12 +1068,13 @@ int Engine::evaluate(int neq, const float* qj, double* vi, double* gxi, double* 
       if ((rc = run_m2l_all(l0))) return rc;
       for (int l = l0 + 1; l <= lmax; l++)
         if ((rc = run_l2l(l, true))) return rc;
-    } else if (far && overlap && !hh && lmax > l0 && m2l_splits(lmax) > 1) {
+    } else if (far && overlap && !hh && lmax > l0 && m2l_partials(lmax)) {
       // levels 2..lmax-1 (M2L, L2L) on the third stream while the leaf M2L
       // computes its partial sums; then the leaf L2L and the reduction that
       // adds the partials (the serialized order below, bit for bit)
       FMMX_HIP(hipEventRecord(ev[12], stream));
       FMMX_HIP(hipStreamWaitEvent(aux2, ev[12], 0));
+      join.side[1] = aux2;
       hipStream_t main = stream;
       stream = aux2;
       part_buf = &m2l_part2;
@@ -1076,6 +1088,7 @@ int Engine::evaluate(int neq, const float* qj, double* vi, double* gxi, double* 
       FMMX_HIP(hipEventRecord(ev[13], aux2));
       if ((rc = run_m2l(lmax, false, 1))) return rc;
       FMMX_HIP(hipStreamWaitEvent(stream, ev[13], 0));
+      join.side[1] = nullptr;
       if ((rc = run_l2l(lmax))) return rc;
       if ((rc = run_m2l(lmax, false, 2))) return rc;
     } else {
@@ -1087,6 +1100,7 @@ int Engine::evaluate(int neq, const float* qj, double* vi, double* gxi, double* 
     }
     if ((rc = mark())) return rc;  // ev6: after M2L+L2L
     if (overlap) FMMX_HIP(hipStreamWaitEvent(stream, ev[11], 0));
+    join.side[0] = nullptr;
     // Laplace and Yukawa: L2P writes the outputs in the caller's order itself
     if (far && (rc = run_l2p(neq, hh ? nullptr : dsts))) return rc;
     if ((rc = mark())) return rc;  // ev7: after L2P

@@ -278,10 +278,13 @@ struct Engine {
   bool last_m2l_all = false;  // the last evaluation took that form
   bool m2l_timed = false;     // the last evaluation recorded ev[8], ev[9] around its M2L launch
   bool m2l_all_levels() const {
-    if (fp64) return orbit_f64();
+    if (fp64 && !orbit_f64()) return false;
     const char* e = getenv("FMMX_M2L_FUSED");
     return !e || atoi(e) != 0;
   }
+  // a level's launch may leave its partial sums for a reduction later on (run_m2l
+  // phases 1 and 2): offset splits, and not by orbits, which reduce with their launch
+  bool m2l_partials(int lev) const { return !orbit_f64() && m2l_variant(lev).pa != 6 && m2l_splits(lev) > 1; }
   M2LLev m2l_desc(int lev, int nt, int wpg, int nsplit, float* part, int init, int wg0);
   int run_l2l(int lev, bool add = false);
   // dst: outputs in the caller's order (v, gx, gy, gz; NULL entries skipped),
