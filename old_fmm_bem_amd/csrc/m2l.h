@@ -313,6 +313,10 @@ struct MSplitLevels {
   unsigned* mmax[MAXL + 1];
   long off[MAXL + 2];
   int nl;
+  // independent groups of boxes (Helmholtz): each has its own scale, mmax[k][key >> 3 gs],
+  // since its potentials do not see the other groups' magnitudes; ng of them (1: none)
+  const uint32_t* key[MAXL + 1];
+  int gs[MAXL + 1], ng;
   int wide;  // 1: layout of the 32x32x16 kernel (WLayout), 2: orbit kernel (OLayout, FP32), else HLayout
 };
 

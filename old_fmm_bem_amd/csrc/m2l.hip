@@ -779,7 +779,10 @@ int Engine::run_m2l_hh(int l0, int l1, bool init) {
   for (int lev = l0; lev <= l1; lev++)
     if (si.nb[lev] > 0 && sj.nb[lev] > 0) need += (size_t)m2l_splits(lev) * si.nb[lev] * rows;
   int rc = m2l_part.ensure(std::max<size_t>(need, 1) * 4);
-  if (rc || (rc = mmax_buf.ensure((MAXL + 1) * 4))) return rc;
+  // one scale per level and independent group
+  const int lg = first_m2l_level();
+  S.ng = group_level > 0 ? 1 << (3 * group_level) : 1;
+  if (rc || (rc = mmax_buf.ensure(std::max<size_t>(MAXL + 1, (size_t)(lmax - lg + 1) * S.ng) * 4))) return rc;
   size_t off = 0;
   int wg = 0;
   for (int lev = l0; lev <= l1; lev++) {
@@ -792,11 +795,13 @@ int Engine::run_m2l_hh(int l0, int l1, bool init) {
     }
     S.M[S.nl] = mexp[lev].as<float>();
     S.Mh[S.nl] = mexp_h[lev].as<uint4>();
-    S.mmax[S.nl] = mmax_buf.as<unsigned>() + lev;
+    S.mmax[S.nl] = mmax_buf.as<unsigned>() + (size_t)(lev - lg) * S.ng;
+    S.key[S.nl] = sj.bkey[lev].as<uint32_t>();
+    S.gs[S.nl] = group_shift(lev);
     S.off[S.nl + 1] = S.off[S.nl] + sj.nb[lev] + 1;
-    S.nl++;
     const int ns = m2l_splits(lev);
     M2LLev& d = A.lv[A.nlv++] = m2l_desc(lev, 1, ORB_WPG, ns, m2l_part.as<float>() + off, init ? 1 : 0, wg);
+    d.mmax = S.mmax[S.nl++];
     d.opH = hop_m2l.as<uint4>() + (size_t)(lev - 2) * NORBOP * frg;
     d.sa_e = hop_e[lev];
     wg += d.nwg;

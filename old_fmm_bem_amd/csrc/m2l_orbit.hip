@@ -51,7 +51,7 @@ __global__ __launch_bounds__(256) void k_morder(MSplitLevels S) {
   const int src = c_otab<P>.src[e];
   float v = 0.f;
   if (b != S.off[k + 1] - 1 && src >= 0)
-    v = S.M[k][(size_t)(b - S.off[k]) * MLayout<P>::VS + src] * ldexpf(1.f, orbit_exp(S.mmax[k]));
+    v = ldexpf(S.M[k][(size_t)(b - S.off[k]) * MLayout<P>::VS + src], orbit_exp(S.mmax[k]));
   reinterpret_cast<float*>(S.Mh[k])[(size_t)(b - S.off[k]) * OC::BS + e] = v;
 }
 
@@ -441,11 +441,12 @@ __global__ __launch_bounds__(ORB_NTH) __attribute__((amdgpu_waves_per_eu(4, 4)))
   group(std::integral_constant<int, 5>{});
   group(std::integral_constant<int, 6>{});
 
-  const float oscale = ldexpf(1.f, -(orbit_exp(Q.mmax) + Q.sa_e));
+  const int oexp = -(orbit_exp(Q.mmax) + Q.sa_e);
   if (tord >= 0) {
     f32x4* dst = reinterpret_cast<f32x4*>(Q.part + ((size_t)split * nb + tord) * OC::ROWS + 4 * kq);
 #pragma unroll
-    for (int c = 0; c < 8; c++) dst[4 * c] = acc[c] * oscale;
+    for (int c = 0; c < 8; c++)
+      dst[4 * c] = f32x4{ldexpf(acc[c][0], oexp), ldexpf(acc[c][1], oexp), ldexpf(acc[c][2], oexp), ldexpf(acc[c][3], oexp)};
   }
   if (mypairs) atomicAdd(Q.npairs, (unsigned long long)mypairs);
 }

@@ -31,37 +31,49 @@ struct GTables {
 template <int P, int HH>
 __constant__ GTables<P, HH> c_gtab = GTables<P, HH>();
 
-// largest |multipole| of every level (float bits; zeroed before), 8 floats per
-// thread: a box is PARTS padded vectors, whose pads are zero
+// scale word of box b of the flattened range, in level k
+__device__ __forceinline__ unsigned* scale_word(const MSplitLevels& S, int k, long b) {
+  return S.mmax[k] + (S.ng > 1 ? S.key[k][b - S.off[k]] >> (3 * S.gs[k]) : 0u);
+}
+
+// largest |multipole| of every level and group (float bits; zeroed before), 8 floats
+// per thread: a box is PARTS padded vectors, whose pads are zero.  Waves and
+// workgroups within one scale word reduce before the global atomic.
 template <int P, int HH>
 __global__ __launch_bounds__(256) void k_gmax(MSplitLevels S) {
   constexpr int N8 = GConst<P, HH>::PARTS * MLayout<P>::VS / 8;
   const long t = (long)blockIdx.x * 256 + threadIdx.x, b = t / N8;
-  __shared__ unsigned smax[MAXL + 1];
-  if (threadIdx.x <= MAXL) smax[threadIdx.x] = 0u;
-  __syncthreads();
+  __shared__ unsigned smax;
+  __shared__ unsigned* sword;
   int k = 0;
   while (k + 1 < S.nl && b >= S.off[k + 1]) k++;
   float mx = 0.f;
+  unsigned* word = S.mmax[k];
   if (b < S.off[S.nl] && b != S.off[k + 1] - 1) {
     const f32x4* m = reinterpret_cast<const f32x4*>(S.M[k]) + ((size_t)(b - S.off[k]) * N8 + t % N8) * 2;
     const f32x4 u = m[0], v = m[1];
 #pragma unroll
     for (int e = 0; e < 4; e++) mx = fmaxf(mx, fmaxf(fabsf(u[e]), fabsf(v[e])));
+    word = scale_word(S, k, b);
   }
-  // a wave within one level reduces first
-  const int k0 = __builtin_amdgcn_readfirstlane(k);
-  if (__ballot(k != k0) == 0) {
-    for (int d = 32; d > 0; d >>= 1) mx = fmaxf(mx, __shfl_xor(mx, d));
-    if ((threadIdx.x & 63) == 0 && mx > 0.f) atomicMax(&smax[k0], __float_as_uint(mx));
-  } else if (mx > 0.f) {
-    atomicMax(&smax[k], __float_as_uint(mx));
+  if (threadIdx.x == 0) {
+    smax = 0u;
+    sword = word;
   }
   __syncthreads();
-  if ((int)threadIdx.x < S.nl && smax[threadIdx.x]) atomicMax(S.mmax[threadIdx.x], smax[threadIdx.x]);
+  unsigned* const mine = sword;
+  if (__ballot(word != mine) == 0) {
+    for (int d = 32; d > 0; d >>= 1) mx = fmaxf(mx, __shfl_xor(mx, d));
+    if ((threadIdx.x & 63) == 0 && mx > 0.f) atomicMax(&smax, __float_as_uint(mx));
+  } else if (mx > 0.f) {
+    atomicMax(word == mine ? &smax : word, __float_as_uint(mx));
+  }
+  __syncthreads();
+  if (threadIdx.x == 0 && smax) atomicMax(mine, smax);
 }
-__global__ void k_gzero(MSplitLevels S) {
-  if ((int)threadIdx.x < S.nl) *S.mmax[threadIdx.x] = 0u;
+__global__ __launch_bounds__(256) void k_gzero(MSplitLevels S) {
+  const unsigned t = blockIdx.x * 256 + threadIdx.x;
+  if (t < (unsigned)(S.nl * S.ng)) S.mmax[t / S.ng][t % S.ng] = 0u;
 }
 
 // multipoles of every level in the stored layout, scaled (as k_morder)
@@ -77,7 +89,7 @@ __global__ __launch_bounds__(256) void k_gorder(MSplitLevels S) {
   const int src = c_gtab<P, HH>.src[e];
   float v = 0.f;
   if (b != S.off[k + 1] - 1 && src >= 0)
-    v = S.M[k][(size_t)(b - S.off[k]) * G::PARTS * MLayout<P>::VS + src] * ldexpf(1.f, orbit_exp(S.mmax[k]));
+    v = ldexpf(S.M[k][(size_t)(b - S.off[k]) * G::PARTS * MLayout<P>::VS + src], orbit_exp(scale_word(S, k, b)));
   reinterpret_cast<float*>(S.Mh[k])[(size_t)(b - S.off[k]) * G::BS + e] = v;
 }
 
@@ -400,13 +412,15 @@ __global__ __launch_bounds__(GEN_NTH) __attribute__((amdgpu_waves_per_eu(2, 2)))
   group(std::integral_constant<int, 5>{});
   group(std::integral_constant<int, 6>{});
 
-  const float oscale = ldexpf(1.f, -(orbit_exp(Q.mmax) + Q.sa_e));
   if (tord >= 0) {
+    const int oexp = -(orbit_exp(Q.mmax + (gsh >= 0 ? Q.ikey[tord] >> (3 * gsh) : 0u)) + Q.sa_e);
     f32x4* dst = reinterpret_cast<f32x4*>(Q.part + ((size_t)split * nb + tord) * G::ROWS + 4 * kq);
 #pragma unroll
     for (int q = 0; q < PARTS; q++)
 #pragma unroll
-      for (int t = 0; t < NT; t++) dst[4 * (q * NT + t)] = acc[q][t] * oscale;
+      for (int t = 0; t < NT; t++)
+        dst[4 * (q * NT + t)] = f32x4{ldexpf(acc[q][t][0], oexp), ldexpf(acc[q][t][1], oexp), ldexpf(acc[q][t][2], oexp),
+                                      ldexpf(acc[q][t][3], oexp)};
   }
   if (mypairs) atomicAdd(Q.npairs, (unsigned long long)mypairs);
 }
@@ -456,7 +470,7 @@ int launch_orbit_gen_order(int p, int hh, const MSplitLevels& S, hipStream_t str
     constexpr int P = decltype(pc)::value, H = decltype(hc)::value;
     using G = GConst<P, H>;
     const long n = S.off[S.nl] * G::BS, n8 = S.off[S.nl] * (G::PARTS * MLayout<P>::VS / 8);
-    k_gzero<<<1, 64, 0, stream>>>(S);
+    k_gzero<<<(S.nl * S.ng + 255) / 256, 256, 0, stream>>>(S);
     k_gmax<P, H><<<(int)((n8 + 255) / 256), 256, 0, stream>>>(S);
     k_gorder<P, H><<<(int)((n + 255) / 256), 256, 0, stream>>>(S);
     return hipGetLastError() == hipSuccess ? FMMX_OK : fail(FMMX_EDEVICE, "orbit M2L reorder launch failed");

@@ -17,13 +17,15 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-// 2^e that brings the level's largest magnitude just below 2^ORB_TOP
+// e of the power of two that brings a level's (or group's) largest magnitude just
+// below 2^ORB_TOP.  Applied with ldexpf, here and when it is undone: 2^e itself is
+// no FP32 number for magnitudes near the ends of FP32's range.
 __device__ __forceinline__ int orbit_exp(const unsigned* mmax) {
   const float m = __uint_as_float(*mmax);
-  if (!(m > 0.f) || !(m < 3.0e38f)) return 0;
+  if (!(m > 0.f) || !(m < __builtin_inff())) return 0;
   int e;
   (void)frexpf(m, &e);
-  return min(100, max(-100, ORB_TOP - e));
+  return ORB_TOP - e;
 }
 
 // bits of v (0..3) at positions 0 and 3 (one axis of a Morton key)
