@@ -266,8 +266,9 @@ void orbit_gen_fragments(const double* C, const double* S, int ld, int p, int sa
 // the distinct base offsets of the orbits, NORBOP of them
 void orbit_op_vector(int i, int* d);
 
-// largest |multipole| after scaling: sums of 4 stay below 2^15 in FP16
-constexpr int ORB_TOP = 13;
+// exponent that scaled multipoles stay below: sums of 4 reach up to FP16's 65,504, and
+// the dense FP16 forms' resolution (SPLIT_TOP) is kept
+constexpr int ORB_TOP = SPLIT_TOP;
 // base offset of product o for a target of parity class cls (bits x, y, z) and
 // the operator's index in [0, NORBOP)
 void orbit_offset(int o, int cls, int* d);

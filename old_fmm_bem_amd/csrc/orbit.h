@@ -18,14 +18,14 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // e of the power of two that brings a level's (or group's) largest magnitude just
-// below 2^ORB_TOP.  Applied with ldexpf, here and when it is undone: 2^e itself is
+// below 2^ORB_TOP, or half of it where sums of 4 would round beyond FP16's 65,504.  Applied with ldexpf, here and when it is undone: 2^e itself is
 // no FP32 number for magnitudes near the ends of FP32's range.
 __device__ __forceinline__ int orbit_exp(const unsigned* mmax) {
   const float m = __uint_as_float(*mmax);
   if (!(m > 0.f) || !(m < __builtin_inff())) return 0;
   int e;
-  (void)frexpf(m, &e);
-  return ORB_TOP - e;
+  const float f = frexpf(m, &e);
+  return (f <= 65504.f / 65536.f ? ORB_TOP : ORB_TOP - 1) - e;
 }
 
 // bits of v (0..3) at positions 0 and 3 (one axis of a Morton key)

@@ -53,3 +53,30 @@ def test_helmholtz_strengths_near_the_ends_of_fp32(scale):
     vd = _run("fp64", 10, x, (q.astype(np.complex128) * scale).astype(np.complex64), F.HELMHOLTZ)
     print(scale, rel_l2(vm / scale, vd / scale), flush=True)
     assert rel_l2(vm / scale, vd / scale) < 5e-6
+
+
+@pytest.mark.parametrize("p", [8, 10])
+def test_laplace_orbits_resolve_as_much_as_the_dense_form(p):
+    """Where FP16's smallest steps are the error (a group 1e-6 weaker than the
+    rest), the orbit form is no further off than the form that multiplies every
+    offset: the same steps, once per sum of up to four sources and not once per
+    source.  A quarter for the scatter of two roundings."""
+    x, q = uniform_cube(20000, 63)
+    weak = x[:, 0] <= 0.5
+    q = np.where(weak, 1e-6 * q, q).astype(np.float32)
+    ref = _run("fp64", p, x, q, F.G, groups=1)[weak]
+    e6, e5 = (rel_l2(_run("mixed", p, x, q, F.G, groups=1, staging=s)[weak], ref) for s in (6, 5))
+    print(p, e6, e5, flush=True)
+    assert e6 < 1.25 * e5
+
+
+@pytest.mark.parametrize("top", [0.99, 0.9995, 0.99999, 1.0])
+def test_sums_at_the_top_of_fp16(top):
+    """Every box alike and its largest multipole at the end of a binade: sums of
+    four sources stay finite in FP16 and keep the engine's accuracy."""
+    k = (np.arange(16) + 0.5) / 16
+    x = np.stack(np.meshgrid(k, k, k, indexing="ij"), -1).reshape(-1, 3).astype(np.float32)
+    q = np.full(len(x), np.float32(top), np.float32)  # one charge per leaf: M_00 = q
+    vm, vd = (_run(prec, 8, x, q, F.G) for prec in ("mixed", "fp64"))
+    print(top, rel_l2(vm, vd), flush=True)
+    assert rel_l2(vm, vd) < 2e-6
