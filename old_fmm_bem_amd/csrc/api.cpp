@@ -500,6 +500,9 @@ void Engine::drop_graph() {
   if (graph) (void)hipGraphDestroy(graph);
   gexec = nullptr;
   graph = nullptr;
+  if (!kept.empty()) (void)hipDeviceSynchronize();
+  for (void* b : kept) (void)hipFree(b);
+  kept.clear();
 }
 
 int Engine::graph_capture(int neq, const float* qj, double* vi, double* gxi, double* gyi, double* gzi) {
@@ -992,6 +995,7 @@ int Engine::prepare(int neq) {
 }
 
 int Engine::evaluate(int neq, const float* qj, double* vi, double* gxi, double* gyi, double* gzi, int flags) {
+  const KeepBlocks keep(*this);
   int rc = check_eval(neq, qj, vi, gxi, gyi, gzi);
   if (rc || (rc = prepare(neq))) return rc;
   const bool dev = flags & FMMX_DEVICE_PTRS;
@@ -1141,6 +1145,7 @@ int Engine::evaluate(int neq, const float* qj, double* vi, double* gxi, double* 
 int Engine::phase(int ph, int neq, int lev, const float* qj, double* vi, double* gxi, double* gyi, double* gzi,
                   int flags) {
   if (neq == FMMX_HELMHOLTZ) return fail(FMMX_EUNSUPPORTED, "phases of the Helmholtz kernel are not provided");
+  const KeepBlocks keep(*this);
   const bool needs_q = ph == FMMX_PHASE_P2P || ph == FMMX_PHASE_P2M;
   const bool writes = ph == FMMX_PHASE_P2P || ph == FMMX_PHASE_L2P;
   if (ph < FMMX_PHASE_P2P || ph > FMMX_PHASE_L2P) return fail(FMMX_EINVAL, "phase out of range [0, 5]");

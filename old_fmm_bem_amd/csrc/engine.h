@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <array>
 #include <memory>
+#include <vector>
 
 #include "fmmx_internal.h"
 
@@ -26,6 +27,9 @@ struct DevBuf {
   void* p = nullptr;
   size_t bytes = 0;
   bool view = false;
+  // set while a captured evaluation exists (Engine::KeepBlocks): blocks that a
+  // buffer leaves are its launches' arguments and live on here
+  static inline thread_local std::vector<void*>* keep = nullptr;
   DevBuf() = default;
   DevBuf(const DevBuf&) = delete;
   DevBuf& operator=(const DevBuf&) = delete;
@@ -48,7 +52,9 @@ struct DevBuf {
       view = false;
     }
     if (need <= bytes && p) return FMMX_OK;
-    if (p) {
+    if (p && keep) {
+      keep->push_back(p);
+    } else if (p) {
       // growing: earlier asynchronous work may still read the old block
       (void)hipDeviceSynchronize();
       (void)hipFree(p);
@@ -183,6 +189,13 @@ struct Engine {
   hipStream_t gstream = nullptr;  // capture and replay stream
   hipEvent_t gev[2] = {};         // orders replays after / before the caller's stream
   bool capturing = false;
+  // blocks of buffers that grew in later evaluations, freed with the graph
+  std::vector<void*> kept;
+  struct KeepBlocks {
+    std::vector<void*>* outer = DevBuf::keep;
+    explicit KeepBlocks(Engine& e) { DevBuf::keep = e.gexec ? &e.kept : nullptr; }
+    ~KeepBlocks() { DevBuf::keep = outer; }
+  };
   void drop_graph();
   int graph_capture(int neq, const float* qj, double* vi, double* gxi, double* gyi, double* gzi);
   int graph_launch();
