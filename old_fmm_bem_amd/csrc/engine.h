@@ -66,6 +66,13 @@ struct DevBuf {
     bytes = b;
     return FMMX_OK;
   }
+  // before new contents that a captured evaluation must not see: another block
+  void renew() {
+    if (!keep || !p || view) return;
+    keep->push_back(p);
+    p = nullptr;
+    bytes = 0;
+  }
   template <class T>
   T* as() const { return static_cast<T*>(p); }
 };

@@ -446,7 +446,11 @@ int Engine::run_p2p(int neq) {
   const double now[2] = {es ? atof(es) : P2P_SMALL, es ? 1.0 : 0.0};
   int rc = FMMX_OK;
   if (now[0] != p2p_bound[0] || now[1] != p2p_bound[1]) {
-    // the bound changed since the items were built
+    // the bound changed since the items were built (a captured evaluation's
+    // launches keep theirs)
+    p2p_items.renew();
+    p2p_count.renew();
+    if ((rc = p2p_count.ensure(4))) return rc;
     k_zero_i<<<1, 64, 0, stream>>>(p2p_count.as<int>());
     if ((rc = build_p2p_items())) return rc;
   }

@@ -78,3 +78,23 @@ def test_the_bound_changes_between_evaluations(monkeypatch, prec):
         print(prec, small, flush=True)
         assert rel_l2(f.evaluate(q)[0], d) < (2e-6 if prec == "mixed" else 1e-13)
     f.close()
+
+
+def test_a_captured_evaluation_keeps_its_items(monkeypatch):
+    torch = pytest.importorskip("torch")
+    x, rng = _points(LANES256, 7)
+    xd = torch.from_numpy(x).cuda()
+    qd = torch.from_numpy(rng.uniform(-1, 1, len(x)).astype(np.float32)).cuda()
+    f = _engine("mixed")
+    f.set_points(xd)
+    want = f.evaluate(qd)[0].clone()
+    v, _ = f.capture(qd)
+    for rep, small in enumerate(("1", "1000", "1")):
+        monkeypatch.setenv("FMMX_P2P_SMALL", small)
+        f.evaluate(qd)
+        v.zero_()
+        torch.cuda.synchronize()
+        f.replay()
+        f.synchronize()
+        assert torch.equal(v, want), rep
+    f.close()
