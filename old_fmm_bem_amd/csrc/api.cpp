@@ -190,13 +190,14 @@ struct OpSet {
   std::vector<double> m2l_frag;  // MFMA fragment order (FP32 engine)
   std::vector<double> m2l_canon; // fragment order, the 56 offsets with dx, dy, dz >= 0 (EXACT)
   std::vector<double> m2l_kmaj;  // transposed [op][k][row] (FP64 engine)
-  // FP16 split M2L (EXACT, p 6..12): hi/lo fragments of the 56 canonical
-  // operators scaled by 2^split_e
+  // FP16 split M2L (EXACT, p 6..12), built when an engine first uploads the form
+  // (get_split): hi/lo fragments of the 56 canonical operators scaled by 2^split_e
   std::vector<uint4> m2l_split;
   int split_e = 0;
   // the same split for the 32x32x16 kernel: all 316 operators as they act
   std::vector<uint4> m2l_wide;
-  // the same split for the reflection-orbit kernel: its NORBOP operators
+  // the same split for the reflection-orbit kernel: its NORBOP operators (of the
+  // Helmholtz sets: built with the set)
   std::vector<uint4> m2l_orbit;
   std::vector<double> m2l_orbit_f64;  // the orbit operators of the FP64 engine (get_orbit_f64)
   std::vector<int> lev_e;  // scale exponents of per-level orbit operators
@@ -298,23 +299,36 @@ std::shared_ptr<OpSet> get_ops(const Tables& T, int lmax, float rd) {
       const int oi = offset_index(d[0], d[1], d[2]);
       std::copy(&S->m2l_frag[(size_t)oi * fr], &S->m2l_frag[(size_t)oi * fr] + fr, &S->m2l_canon[(size_t)ci * fr]);
     }
-    if (m2l_split_supported(T.p)) {
-      std::vector<double> ck((size_t)NCANON * sq);
-      for (int ci = 0; ci < NCANON; ci++) {
-        int d[3];
-        canon_vector(ci, d);
-        const int oi = offset_index(d[0], d[1], d[2]);
-        std::copy(&S->m2l_kmaj[(size_t)oi * sq], &S->m2l_kmaj[(size_t)oi * sq] + sq, &ck[(size_t)ci * sq]);
-      }
-      S->split_e = split_scale_exp(ck.data(), ck.size());
-      split_fragments(ck.data(), NCANON, T.p, S->split_e, S->m2l_split);
-      if (m2l_orbit_supported(T.p)) orbit_fragments(S->m2l_kmaj.data(), T.p, S->split_e, S->m2l_orbit);
-      if (split_wide_fits(T.p)) split_fragments_wide(S->m2l_kmaj.data(), NOFF, T.p, S->split_e, S->m2l_wide);
-    }
+    if (m2l_split_supported(T.p)) S->split_e = split_scale_exp(S->m2l_canon.data(), S->m2l_canon.size());
   }
   std::lock_guard<std::mutex> lk(g_cache_mu);
   g_cache[key] = S;
   return S;
+}
+
+// the fragments of an FP16 M2L form of a Laplace set (6 orbits, 5 wide, else split).
+// Each form is built when an engine first takes it: at p = 10 the three cost 72, 313
+// and 56 ms of one host thread, and an evaluation needs one.
+const std::vector<uint4>& get_split(OpSet& S, int p, int form) {
+  std::lock_guard<std::mutex> lk(g_cache_mu);
+  std::vector<uint4>& v = form == 6 ? S.m2l_orbit : form == 5 ? S.m2l_wide : S.m2l_split;
+  if (!v.empty()) return v;
+  if (form == 6) {
+    orbit_fragments(S.m2l_kmaj.data(), p, S.split_e, v);
+  } else if (form == 5) {
+    split_fragments_wide(S.m2l_kmaj.data(), NOFF, p, S.split_e, v);
+  } else {
+    const size_t sq = (size_t)p * p * p * p;
+    std::vector<double> ck((size_t)NCANON * sq);
+    for (int ci = 0; ci < NCANON; ci++) {
+      int d[3];
+      canon_vector(ci, d);
+      const double* A = &S.m2l_kmaj[(size_t)offset_index(d[0], d[1], d[2]) * sq];
+      std::copy(A, A + sq, &ck[(size_t)ci * sq]);
+    }
+    split_fragments(ck.data(), NCANON, p, S.split_e, v);
+  }
+  return v;
 }
 
 // the FP64 orbit fragments of a Laplace set, built when an FP64 engine first asks
@@ -761,9 +775,9 @@ int Engine::upload_operators() {
         (rc = upload<float>(op_m2l, canon ? S->m2l_canon : S->m2l_frag, stream)))
       return rc;
     // the operators of the FP16 form in use go up behind the tree (upload_split)
-    split_ok = canon && !S->m2l_split.empty();
-    wide_ok = split_ok && !S->m2l_wide.empty();
-    orb_ok = split_ok && !S->m2l_orbit.empty();
+    split_ok = canon && m2l_split_supported(p);
+    wide_ok = split_ok && split_wide_fits(p);
+    orb_ok = split_ok && m2l_orbit_supported(p);
     sa_e = S->split_e;
     up_h = up_w = up_o = false;
   }
@@ -777,7 +791,7 @@ int Engine::upload_split(int form) {
   if (up) return FMMX_OK;
   if (capturing) return fail(FMMX_ESTATE, "M2L operators not uploaded before capture");
   auto S = get_ops(tab, ops_lmax, ops_rd);  // built at upload_operators: a lookup
-  const std::vector<uint4>& v = form == 6 ? S->m2l_orbit : form == 5 ? S->m2l_wide : S->m2l_split;
+  const std::vector<uint4>& v = get_split(*S, p, form);
   DevBuf& dst = form == 6 ? op_m2l_o : form == 5 ? op_m2l_w : op_m2l_h;
   int rc = dst.ensure(v.size() * 16);
   if (rc) return rc;
