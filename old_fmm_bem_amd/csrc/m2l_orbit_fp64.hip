@@ -1,6 +1,7 @@
 // m2l_orbit_fp64.hip -- M2L of the FP64 engine by reflection orbits on the FP64
 // matrix cores (Laplace, EXACT, p = 6..12): 63 products per target instead of
 // 189, with the sums over an orbit's sources and all products in FP64.
+#include "mfma.h"
 #include "orbit.h"
 
 namespace fmmx {
@@ -8,7 +9,6 @@ namespace fmmx {
 namespace {
 
 typedef double d2 __attribute__((ext_vector_type(2)));
-typedef double d4 __attribute__((ext_vector_type(4)));
 
 template <int P>
 struct FTables {
@@ -129,9 +129,9 @@ __global__ __launch_bounds__(F64_NTH) __attribute__((amdgpu_waves_per_eu(2, 2)))
       axk[ax][d + 3][w * 16 + j] = ok ? k : 0x80000000u;
     }
   }
-  d4 acc[NT];
+  f64x4 acc[NT];
 #pragma unroll
-  for (int t = 0; t < NT; t++) acc[t] = d4{0., 0., 0., 0.};
+  for (int t = 0; t < NT; t++) acc[t] = Mfma<double>::zero();
   unsigned mypairs = 0;
   const int4* __restrict__ otab = orbtab + cls * NORB;
   uint32_t src[4];  // boxes of the product about to run, in 64-byte units
@@ -308,7 +308,7 @@ __global__ __launch_bounds__(F64_NTH) __attribute__((amdgpu_waves_per_eu(2, 2)))
             for (int h = 0; h < 2; h++) {
               const int kc = XT ? L.qc[(2 * u + h) & 3] : 2 * u + h;
               const int c = sub_rank(D, (L.tcls[t] ^ kc) & D);
-              acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(f[h], raw[c][h], acc[t], 0, 0, 0);
+              acc[t] = Mfma<double>::fma(f[h], raw[c][h], acc[t]);
             }
           }
           __builtin_amdgcn_sched_barrier(0);
@@ -335,7 +335,7 @@ __global__ __launch_bounds__(F64_NTH) __attribute__((amdgpu_waves_per_eu(2, 2)))
 
   // the operators' rows are ordered so that a lane holds four rows in turn
   if (tord >= 0) {
-    d4* dst = reinterpret_cast<d4*>(reinterpret_cast<double*>(Q.part) + ((size_t)split * nb + tord) * F::ROWS + 4 * kq);
+    f64x4* dst = reinterpret_cast<f64x4*>(reinterpret_cast<double*>(Q.part) + ((size_t)split * nb + tord) * F::ROWS + 4 * kq);
 #pragma unroll
     for (int t = 0; t < NT; t++) dst[4 * t] = acc[t];
   }

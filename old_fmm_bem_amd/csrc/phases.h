@@ -9,6 +9,7 @@
 
 #include "engine.h"
 #include "m2l.h"
+#include "mfma.h"
 #include "tree_util.h"
 
 namespace fmmx {
@@ -240,26 +241,6 @@ __device__ __forceinline__ void box_center(uint32_t key, int lev, double xmin, d
   cy = ymin + (iy + 0.5) * rb;
   cz = zmin + (iz + 0.5) * rb;
 }
-
-// v_mfma 16x16x4 in FP32 and FP64
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef double f64x4 __attribute__((ext_vector_type(4)));
-template <typename T>
-struct Mfma;
-template <>
-struct Mfma<float> {
-  using v4 = f32x4;
-  static __device__ __forceinline__ v4 fma(float a, float b, v4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-};
-template <>
-struct Mfma<double> {
-  using v4 = f64x4;
-  static __device__ __forceinline__ v4 fma(double a, double b, v4 c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-};
 
 template <typename T>
 __global__ void k_m2l_reduce(long n, int nsplit, const T* __restrict__ part, T* __restrict__ L, int init) {

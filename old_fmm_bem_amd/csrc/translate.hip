@@ -192,12 +192,7 @@ __global__ __launch_bounds__(L2L ? 256 : 512) void k_translate_mfma(int nout, co
   }
   V4 acc[MT];
 #pragma unroll
-  for (int mt = 0; mt < MT; mt++) {
-    acc[mt] = V4{T(0), T(0), T(0), T(0)};
-    // zeros in registers: with a constant zero for its accumulator the compiler
-    // may give an FP64 MFMA an output that overlaps its own operands
-    if constexpr (D) asm volatile("" : "+v"(acc[mt]));
-  }
+  for (int mt = 0; mt < MT; mt++) acc[mt] = Mfma<T>::zero();
   if (__ballot(src >= 0) != 0) {
     T bv[KS];
     if (L2L) {

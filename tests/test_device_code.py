@@ -69,3 +69,25 @@ def test_lds_copies_wait_for_m0(listing):
                     bad.append((name, prev, ins))
     assert copies > 0
     assert not bad, (len(bad), copies, bad[:3])
+
+
+def _span(operand):
+    """(file, first, last) of a register operand, None for a constant"""
+    m = re.match(r"([av])(?:\[(\d+):(\d+)\]|(\d+))$", operand.strip().split(" ")[0])
+    return m and (m.group(1), int(m.group(2) or m.group(4)), int(m.group(3) or m.group(4)))
+
+
+def test_fp64_mfma_outputs_leave_their_operands_alone(listing):
+    """v_mfma_f64_16x16x4 writes its output while it still reads its operands:
+    they must not share registers."""
+    seen, bad = set(), []
+    for name, code in listing.items():
+        for ins in code:
+            if not ins.startswith("v_mfma_f64_16x16x4"):
+                continue
+            seen.add(name)
+            d, a, b = (_span(o) for o in ins.split(None, 1)[1].split(",")[:3])
+            if any(o and o[0] == d[0] and o[1] <= d[2] and d[1] <= o[2] for o in (a, b)):
+                bad.append((name, ins))
+    assert any("k_m2l_of" in k for k in seen) and any("k_translate_mfma" in k for k in seen)
+    assert not bad, bad[:3]
