@@ -429,7 +429,7 @@ std::shared_ptr<OpSet> get_hh_ops(int p, double k, float rd, int lmax, bool fp64
   S->nlev = lmax - 1;
   const size_t sq = (size_t)P2 * P2, fr = (size_t)((P2 + 3) / 4) * ((P2 + 15) / 16) * 64;
   const int noff = fp64 ? NOFF : NORBOP;
-  const size_t frg = orbit_gen_frags(p, 1);
+  const size_t frg = orbit_gen_frags(p);
   std::vector<double> cs;  // FP32: C and S per (level, base offset)
   if (fp64) {
     S->m2m.assign((size_t)nt_lev * 8 * vq, 0.0);
@@ -998,7 +998,7 @@ int Engine::prepare(int neq) {
     if ((rc = mexp[l].ensure((size_t)std::max(1, sj.nb[l]) * VS * np * es)) ||
         (rc = lexp[l].ensure((size_t)std::max(1, si.nb[l]) * P2 * np * es)))
       return rc;
-    if (hh && !fp64 && (rc = mexp_h[l].ensure((size_t)(sj.nb[l] + 1) * orbit_gen_box_floats(p, 1) * 4))) return rc;
+    if (hh && !fp64 && (rc = mexp_h[l].ensure((size_t)(sj.nb[l] + 1) * orbit_gen_box_floats(p) * 4))) return rc;
     if (orbit_f64() && (rc = mexp_h[l].ensure((size_t)(sj.nb[l] + 1) * orbit_f64_box(p) * 8))) return rc;
     if (split_ok && !hh && !fp64 && (rc = mexp_h[l].ensure((size_t)(sj.nb[l] + 1) * split_box_halfs(p) * 2)))
       return rc;

@@ -178,8 +178,8 @@ struct OConst {
 // The general form (m2l_orbit_gen.hip): row classes of more than 16 slots take
 // two 16-row tiles, and classes of more words than the octets hold put up to
 // two more words of each into one last octet (positions t, t + 4: words NO,
-// NO + 1 of class qc[t]).  HH: Helmholtz, split expansions of two parts, whose
-// operator is [[C, -S], [S, C]] for two real operators C and S.
+// NO + 1 of class qc[t]), for Helmholtz (GConst: split expansions of two parts,
+// whose operator is [[C, -S], [S, C]] for two real operators C and S) and FP64 (FConst).
 template <int P>
 struct GLayout {
   OLayout<P> O;
@@ -217,10 +217,10 @@ struct GLayout {
     return m < O.size[cls(s, t)] ? m : -1;
   }
 };
-template <int P, int HH>
+template <int P>
 struct GConst {
   static constexpr GLayout<P> L{};
-  static constexpr int P2 = P * P, PARTS = HH ? 2 : 1, NO = L.no, XTRA = L.xtra, NSTEP = NO + XTRA, NT = L.nt;
+  static constexpr int P2 = P * P, PARTS = 2, NO = L.no, XTRA = L.xtra, NSTEP = NO + XTRA, NT = L.nt;
   static constexpr int PBS = NSTEP * 32, BS = PARTS * PBS;  // floats of a stored part, box
   static constexpr int CH = NT * PARTS * 2 * 64, FRO = NSTEP * CH;  // 16-byte fragments of a step, operator
   static constexpr int ROWS = PARTS * NT * 16;                      // partial sums per target
@@ -253,15 +253,15 @@ size_t orbit_f64_rows(int p);  // partial sums per target
 // fragments of the NORBOP operators from all 316 k-major ones
 void orbit_f64_fragments(const double* kmaj, int p, std::vector<double>& out);
 
-// launchers of the general form; opset[lev]: fragments of that level's operators
-int launch_m2l_orbit_gen(int p, int hh, const M2LLaunch& A, int nwg, const int4* orbtab, hipStream_t stream);
-int launch_orbit_gen_order(int p, int hh, const MSplitLevels& S, hipStream_t stream);
-int launch_orbit_gen_reduce(int p, int hh, const M2LLaunch& A, hipStream_t stream);
-size_t orbit_gen_box_floats(int p, int hh);
-size_t orbit_gen_frags(int p, int hh);
-size_t orbit_gen_rows(int p, int hh);
-// fragments of one operator (C, and S for hh; row-major P2 x P2 blocks of leading
-// dimension ld), scaled by 2^sa_e
+// launchers of the Helmholtz form (p = 4, 6, 8, 10, 12)
+int launch_m2l_orbit_gen(int p, const M2LLaunch& A, int nwg, const int4* orbtab, hipStream_t stream);
+int launch_orbit_gen_order(int p, const MSplitLevels& S, hipStream_t stream);
+int launch_orbit_gen_reduce(int p, const M2LLaunch& A, hipStream_t stream);
+size_t orbit_gen_box_floats(int p);
+size_t orbit_gen_frags(int p);
+size_t orbit_gen_rows(int p);
+// fragments of one operator (C and S; row-major P2 x P2 blocks of leading dimension
+// ld), scaled by 2^sa_e
 void orbit_gen_fragments(const double* C, const double* S, int ld, int p, int sa_e, uint4* out);
 // the distinct base offsets of the orbits, NORBOP of them
 void orbit_op_vector(int i, int* d);
@@ -278,7 +278,6 @@ bool m2l_orbit_supported(int p);
 // scaled by 2^sa_e: per operator [octet][row class][hi, lo][lane], then the quad
 // step's [row class][lane] with hi and lo in one fragment
 void orbit_fragments(const double* kmaj, int p, int sa_e, std::vector<uint4>& out);
-size_t orbit_frag_count(int p);
 
 // One M2L launch can cover several levels: workgroups [wg0, wg0 + nwg) of
 // the grid run level `lev` with that level's tiles, splits and buffers.

@@ -578,12 +578,12 @@ Engine::M2LVariant Engine::m2l_variant(int lev) const {
       // 0.331 ms for the launch, 16 splits 0.341; a sphere's leaf level of
       // 4,639 boxes 0.104 against 0.125)
       if (v.pa == 6 && tpc > 1) v.nsplit = std::min(v.nsplit, 8);
-      // Helmholtz: one workgroup per CU and 1.5 KB of partial sums per target
-      // and split (sphere of 1M points: 4 splits of the leaf level 1.68 ms for
-      // M2L and L2L, 7 splits 1.84, 2 splits 1.85)
       // FP64 orbits: 512 workgroups of a level, each with its own share of the
       // 63 products (one workgroup per CU at a time)
       if (orbit_f64()) v.nsplit = 512 / (8 * tpc);
+      // Helmholtz: one workgroup per CU and 1.5 KB of partial sums per target
+      // and split (sphere of 1M points: 4 splits of the leaf level 1.68 ms for
+      // M2L and L2L, 7 splits 1.84, 2 splits 1.85)
       if (hh) v.nsplit = std::max(1, std::min(640 / (8 * tpc), tpc > 1 ? 8 : 16));
     }
   }
@@ -591,10 +591,7 @@ Engine::M2LVariant Engine::m2l_variant(int lev) const {
   return v;
 }
 
-// phase 0: the M2L launch and (with splits) the reduction into the locals;
-// 1: the launch alone, partial sums only (needs m2l_splits(lev) > 1);
-// 2: the reduction alone, adding the partials of phase 1 to the locals
-// FP32 MFMA M2L: the launch parameters of one level, its workgroups from wg0
+// MFMA M2L: the launch parameters of one level, its workgroups from wg0
 // (grid = 8 classes x tiles x splits; a block of tiles per XCD once every XCD
 // gets at least one tile)
 M2LLev Engine::m2l_desc(int lev, int nt, int wpg, int nsplit, float* part, int init, int wg0) {
@@ -660,10 +657,6 @@ void launch_m2l(const M2LLaunch& A, int nwg, int nt, int pa, int wpg, hipStream_
 #undef FMMX_M2L_LAUNCH
 }
 
-// FP32 MFMA M2L of all levels l0..lmax in one launch, in the leaf level's
-// launch shape with each level's offset splits: levels with splits write
-// partial sums (reduced afterwards in fixed order), the others write their
-// locals; the L2L chain then adds the parents' locals level by level.
 // the orbit kernel addresses a level's stored boxes with 32-bit byte offsets
 bool Engine::orbit_fits() const { return ((size_t)sj.nb[lmax] + 1) * orbit_box_floats(p) * 4 < ((size_t)1 << 32); }
 
@@ -774,7 +767,7 @@ int Engine::run_m2l_all(int l0) {
 int Engine::run_m2l_hh(int l0, int l1, bool init) {
   M2LLaunch A{};
   MSplitLevels S{};
-  const size_t rows = orbit_gen_rows(p, 1), frg = orbit_gen_frags(p, 1);
+  const size_t rows = orbit_gen_rows(p), frg = orbit_gen_frags(p);
   size_t need = 0;
   for (int lev = l0; lev <= l1; lev++)
     if (si.nb[lev] > 0 && sj.nb[lev] > 0) need += (size_t)m2l_splits(lev) * si.nb[lev] * rows;
@@ -808,9 +801,9 @@ int Engine::run_m2l_hh(int l0, int l1, bool init) {
     off += (size_t)ns * nb * rows;
   }
   if (A.nlv == 0) return FMMX_OK;
-  if ((rc = launch_orbit_gen_order(p, 1, S, stream))) return rc;
-  if ((rc = launch_m2l_orbit_gen(p, 1, A, wg, orbtab.as<int4>(), stream))) return rc;
-  return launch_orbit_gen_reduce(p, 1, A, stream);
+  if ((rc = launch_orbit_gen_order(p, S, stream))) return rc;
+  if ((rc = launch_m2l_orbit_gen(p, A, wg, orbtab.as<int4>(), stream))) return rc;
+  return launch_orbit_gen_reduce(p, A, stream);
 }
 
 // FP64 Laplace M2L of levels l0..l1 by reflection orbits, one launch; the locals
@@ -851,6 +844,9 @@ int Engine::run_m2l_f64(int l0, int l1, bool init) {
   return launch_m2l_orbit_f64(p, S, A, wg, orbtab.as<int4>(), tmark ? ev[8] : nullptr, tmark ? ev[9] : nullptr, stream);
 }
 
+// phase 0: the M2L launch and (with splits) the reduction into the locals;
+// 1: the launch alone, partial sums only (needs m2l_splits(lev) > 1);
+// 2: the reduction alone, adding the partials of phase 1 to the locals
 int Engine::run_m2l(int lev, bool init, int phase) {
   const int nb = si.nb[lev];
   if (nb == 0) return FMMX_OK;

@@ -1,17 +1,16 @@
-// m2l_orbit_gen.hip -- M2L by reflection orbits for the orders and kernels that
-// m2l_orbit.hip does not cover: the Helmholtz kernel of the FP32 engine (split
-// expansions of two parts, row classes of up to 21 slots at p = 12), on the
-// FP16 matrix cores with error compensation (hi/lo operands, three products,
-// FP32 accumulation).
+// m2l_orbit_gen.hip -- M2L by reflection orbits of the FP32 engine's Helmholtz
+// kernel (split expansions of two parts, row classes of up to 21 slots at
+// p = 12), on the FP16 matrix cores with error compensation (hi/lo operands,
+// three products, FP32 accumulation).
 #include "orbit.h"
 
 namespace fmmx {
 
 namespace {
 
-template <int P, int HH>
+template <int P>
 struct GTables {
-  using G = GConst<P, HH>;
+  using G = GConst<P>;
   int16_t src[G::BS];
   int16_t pos[G::PARTS * G::P2];
   constexpr GTables() : src{}, pos{} {
@@ -28,8 +27,8 @@ struct GTables {
             pos[part * G::P2 + L.O.slot[L.tcls[tl]][L.trow[tl] + r]] = (int16_t)((part * G::NT + tl) * 16 + r);
   }
 };
-template <int P, int HH>
-__constant__ GTables<P, HH> c_gtab = GTables<P, HH>();
+template <int P>
+__constant__ GTables<P> c_gtab = GTables<P>();
 
 // scale word of box b of the flattened range, in level k
 __device__ __forceinline__ unsigned* scale_word(const MSplitLevels& S, int k, long b) {
@@ -39,9 +38,9 @@ __device__ __forceinline__ unsigned* scale_word(const MSplitLevels& S, int k, lo
 // largest |multipole| of every level and group (float bits; zeroed before), 8 floats
 // per thread: a box is PARTS padded vectors, whose pads are zero.  Waves and
 // workgroups within one scale word reduce before the global atomic.
-template <int P, int HH>
+template <int P>
 __global__ __launch_bounds__(256) void k_gmax(MSplitLevels S) {
-  constexpr int N8 = GConst<P, HH>::PARTS * MLayout<P>::VS / 8;
+  constexpr int N8 = GConst<P>::PARTS * MLayout<P>::VS / 8;
   const long t = (long)blockIdx.x * 256 + threadIdx.x, b = t / N8;
   __shared__ unsigned smax;
   __shared__ unsigned* sword;
@@ -77,16 +76,16 @@ __global__ __launch_bounds__(256) void k_gzero(MSplitLevels S) {
 }
 
 // multipoles of every level in the stored layout, scaled (as k_morder)
-template <int P, int HH>
+template <int P>
 __global__ __launch_bounds__(256) void k_gorder(MSplitLevels S) {
-  using G = GConst<P, HH>;
+  using G = GConst<P>;
   const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
   const long b = (long)(t / G::BS);
   const int e = (int)(t % G::BS);
   if (b >= S.off[S.nl]) return;
   int k = 0;
   while (k + 1 < S.nl && b >= S.off[k + 1]) k++;
-  const int src = c_gtab<P, HH>.src[e];
+  const int src = c_gtab<P>.src[e];
   float v = 0.f;
   if (b != S.off[k + 1] - 1 && src >= 0)
     v = ldexpf(S.M[k][(size_t)(b - S.off[k]) * G::PARTS * MLayout<P>::VS + src], orbit_exp(scale_word(S, k, b)));
@@ -110,14 +109,14 @@ constexpr int GEN_NTH = 64 * ORB_WPG, GEN_TN = 16 * ORB_WPG;
 // waited for before its products).  Taking products without any source in the
 // workgroup off its list beforehand gained nothing: few are empty for 128
 // targets.
-template <int P, int HH>
+template <int P>
 __global__ __launch_bounds__(GEN_NTH) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_m2l_og(
     M2LLaunch A, const int4* __restrict__ orbtab) {
   M2LLev Q = A.lv[0];
 #pragma unroll
   for (int k = 1; k < MAXL + 1; k++)
     if (k < A.nlv && (int)blockIdx.x >= A.lv[k].wg0) Q = A.lv[k];
-  using G = GConst<P, HH>;
+  using G = GConst<P>;
   constexpr int NSTEP = G::NSTEP, NT = G::NT, PARTS = G::PARTS, CH = G::CH, FRO = G::FRO;
   constexpr GLayout<P> L{};
   const int lev = Q.lev, nb = Q.nb, nbj = Q.nbj, nsplit = Q.nsplit, gsh = Q.gsh;
@@ -376,19 +375,14 @@ __global__ __launch_bounds__(GEN_NTH) __attribute__((amdgpu_waves_per_eu(2, 2)))
           const u32x4 vh = bh[c], vl = bl[c];
           const h8 hi = __builtin_bit_cast(h8, vh), lo = __builtin_bit_cast(h8, vl);
           acc[part][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fh[0], hi, acc[part][t], 0, 0, 0);
-          if constexpr (PARTS == 2) {
-            // Im += S R; Re -= S I: the operand's sign bits
-            const uint32_t sg = part ? 0x80008000u : 0u;
-            const h8 hs = part ? __builtin_bit_cast(h8, vh ^ sg) : hi, ls = part ? __builtin_bit_cast(h8, vl ^ sg) : lo;
-            acc[1 - part][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fh[1], hs, acc[1 - part][t], 0, 0, 0);
-            acc[part][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fl[0], hi, acc[part][t], 0, 0, 0);
-            acc[1 - part][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fl[1], hs, acc[1 - part][t], 0, 0, 0);
-            acc[part][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fh[0], lo, acc[part][t], 0, 0, 0);
-            acc[1 - part][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fh[1], ls, acc[1 - part][t], 0, 0, 0);
-          } else {
-            acc[part][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fl[0], hi, acc[part][t], 0, 0, 0);
-            acc[part][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fh[0], lo, acc[part][t], 0, 0, 0);
-          }
+          // Im += S R; Re -= S I: the operand's sign bits
+          const uint32_t sg = part ? 0x80008000u : 0u;
+          const h8 hs = part ? __builtin_bit_cast(h8, vh ^ sg) : hi, ls = part ? __builtin_bit_cast(h8, vl ^ sg) : lo;
+          acc[1 - part][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fh[1], hs, acc[1 - part][t], 0, 0, 0);
+          acc[part][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fl[0], hi, acc[part][t], 0, 0, 0);
+          acc[1 - part][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fl[1], hs, acc[1 - part][t], 0, 0, 0);
+          acc[part][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fh[0], lo, acc[part][t], 0, 0, 0);
+          acc[1 - part][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fh[1], ls, acc[1 - part][t], 0, 0, 0);
           __builtin_amdgcn_sched_barrier(0);
         }
       }
@@ -433,9 +427,9 @@ struct GReduce {
   int nsplit[MAXL + 1], nb[MAXL + 1], init[MAXL + 1];
   int nl;
 };
-template <int P, int HH>
+template <int P>
 __global__ __launch_bounds__(256) void k_gen_reduce(GReduce R) {
-  using G = GConst<P, HH>;
+  using G = GConst<P>;
   constexpr int N = G::PARTS * G::P2;
   const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
   const unsigned b = (unsigned)(t / N);
@@ -444,7 +438,7 @@ __global__ __launch_bounds__(256) void k_gen_reduce(GReduce R) {
   int k = 0;
   while (k + 1 < R.nl && b >= R.off[k + 1]) k++;
   const unsigned bl = b - R.off[k];
-  const float* p = R.part[k] + (size_t)bl * G::ROWS + c_gtab<P, HH>.pos[i];
+  const float* p = R.part[k] + (size_t)bl * G::ROWS + c_gtab<P>.pos[i];
   float* L = R.L[k] + (size_t)bl * N + i;
   float s = R.init[k] ? 0.f : *L;
   for (int q = 0; q < R.nsplit[k]; q++) s += p[(size_t)q * R.nb[k] * G::ROWS];
@@ -452,12 +446,12 @@ __global__ __launch_bounds__(256) void k_gen_reduce(GReduce R) {
 }
 
 template <typename F>
-int dispatch_gen(int p, int hh, F&& f) {
-  switch (2 * p + (hh ? 1 : 0)) {
-#define FMMX_CASE(P, H) \
-  case 2 * P + H:       \
-    return f(std::integral_constant<int, P>{}, std::integral_constant<int, H>{});
-    FMMX_CASE(4, 1) FMMX_CASE(6, 1) FMMX_CASE(8, 1) FMMX_CASE(10, 1) FMMX_CASE(12, 1)
+int dispatch_gen(int p, F&& f) {
+  switch (p) {
+#define FMMX_CASE(P) \
+  case P:            \
+    return f(std::integral_constant<int, P>{});
+    FMMX_CASE(4) FMMX_CASE(6) FMMX_CASE(8) FMMX_CASE(10) FMMX_CASE(12)
 #undef FMMX_CASE
   }
   return fail(FMMX_EUNSUPPORTED, "order without an orbit M2L");
@@ -465,28 +459,28 @@ int dispatch_gen(int p, int hh, F&& f) {
 
 }  // namespace
 
-int launch_orbit_gen_order(int p, int hh, const MSplitLevels& S, hipStream_t stream) {
-  return dispatch_gen(p, hh, [&](auto pc, auto hc) -> int {
-    constexpr int P = decltype(pc)::value, H = decltype(hc)::value;
-    using G = GConst<P, H>;
+int launch_orbit_gen_order(int p, const MSplitLevels& S, hipStream_t stream) {
+  return dispatch_gen(p, [&](auto pc) -> int {
+    constexpr int P = decltype(pc)::value;
+    using G = GConst<P>;
     const long n = S.off[S.nl] * G::BS, n8 = S.off[S.nl] * (G::PARTS * MLayout<P>::VS / 8);
     k_gzero<<<(S.nl * S.ng + 255) / 256, 256, 0, stream>>>(S);
-    k_gmax<P, H><<<(int)((n8 + 255) / 256), 256, 0, stream>>>(S);
-    k_gorder<P, H><<<(int)((n + 255) / 256), 256, 0, stream>>>(S);
+    k_gmax<P><<<(int)((n8 + 255) / 256), 256, 0, stream>>>(S);
+    k_gorder<P><<<(int)((n + 255) / 256), 256, 0, stream>>>(S);
     return hipGetLastError() == hipSuccess ? FMMX_OK : fail(FMMX_EDEVICE, "orbit M2L reorder launch failed");
   });
 }
 
-int launch_m2l_orbit_gen(int p, int hh, const M2LLaunch& A, int nwg, const int4* orbtab, hipStream_t stream) {
-  return dispatch_gen(p, hh, [&](auto pc, auto hc) -> int {
-    k_m2l_og<decltype(pc)::value, decltype(hc)::value><<<nwg, GEN_NTH, 0, stream>>>(A, orbtab);
+int launch_m2l_orbit_gen(int p, const M2LLaunch& A, int nwg, const int4* orbtab, hipStream_t stream) {
+  return dispatch_gen(p, [&](auto pc) -> int {
+    k_m2l_og<decltype(pc)::value><<<nwg, GEN_NTH, 0, stream>>>(A, orbtab);
     return hipGetLastError() == hipSuccess ? FMMX_OK : fail(FMMX_EDEVICE, "orbit M2L launch failed");
   });
 }
 
-int launch_orbit_gen_reduce(int p, int hh, const M2LLaunch& A, hipStream_t stream) {
-  return dispatch_gen(p, hh, [&](auto pc, auto hc) -> int {
-    constexpr int P = decltype(pc)::value, H = decltype(hc)::value;
+int launch_orbit_gen_reduce(int p, const M2LLaunch& A, hipStream_t stream) {
+  return dispatch_gen(p, [&](auto pc) -> int {
+    constexpr int P = decltype(pc)::value;
     GReduce R{};
     for (int k = 0; k < A.nlv; k++) {
       const M2LLev& d = A.lv[k];
@@ -498,8 +492,8 @@ int launch_orbit_gen_reduce(int p, int hh, const M2LLaunch& A, hipStream_t strea
       R.off[k + 1] = R.off[k] + (unsigned)d.nb;
       R.nl++;
     }
-    const long n = (long)R.off[R.nl] * GConst<P, H>::PARTS * P * P;
-    k_gen_reduce<P, H><<<(int)((n + 255) / 256), 256, 0, stream>>>(R);
+    const long n = (long)R.off[R.nl] * GConst<P>::PARTS * P * P;
+    k_gen_reduce<P><<<(int)((n + 255) / 256), 256, 0, stream>>>(R);
     return hipGetLastError() == hipSuccess ? FMMX_OK : fail(FMMX_EDEVICE, "orbit M2L reduction launch failed");
   });
 }

@@ -167,10 +167,6 @@ int orbit_op_index(const int* d) {
   return it == u.end() ? -1 : (int)(it - u.begin());
 }
 
-size_t orbit_frag_count(int p) {
-  return with_orbit_p(p, [](auto oc, auto) -> size_t { return decltype(oc)::FRO; });
-}
-
 size_t orbit_box_floats(int p) {
   if (!m2l_orbit_supported(p)) return 0;
   return with_orbit_p(p, [](auto oc, auto) -> size_t { return decltype(oc)::BS; });
@@ -221,28 +217,27 @@ void orbit_op_vector(int i, int* d) {
 }
 
 namespace {
-template <int P, int HH>
+template <int P>
 size_t gen_size(int what) {
-  using G = GConst<P, HH>;
+  using G = GConst<P>;
   return what == 0 ? G::BS : what == 1 ? G::FRO : G::ROWS;
 }
-size_t gen_size(int p, int hh, int what) {
-  switch (2 * p + (hh ? 1 : 0)) {
-    case 9: return gen_size<4, 1>(what);
-    case 13: return gen_size<6, 1>(what);
-    case 17: return gen_size<8, 1>(what);
-    case 21: return gen_size<10, 1>(what);
-    case 25: return gen_size<12, 1>(what);
+size_t gen_size(int p, int what) {
+  switch (p) {
+    case 4: return gen_size<4>(what);
+    case 6: return gen_size<6>(what);
+    case 8: return gen_size<8>(what);
+    case 10: return gen_size<10>(what);
+    case 12: return gen_size<12>(what);
   }
   return 0;
 }
 template <int P>
 void gen_fragments(const double* C, const double* S, int ld, int sa_e, uint4* out) {
   constexpr GLayout<P> L{};
-  const int mats = S ? 2 : 1;
   for (int s = 0; s < L.no + L.xtra; s++)
     for (int tl = 0; tl < L.nt; tl++)
-      for (int q = 0; q < mats; q++)
+      for (int q = 0; q < 2; q++)
         for (int l = 0; l < 64; l++) {
           const double* A = q ? S : C;
           const int r = L.trow[tl] + (l & 15), i = r < L.O.size[L.tcls[tl]] ? L.O.slot[L.tcls[tl]][r] : -1;
@@ -255,16 +250,16 @@ void gen_fragments(const double* C, const double* S, int ld, int sa_e, uint4* ou
             h[1][t] = to_half(a - from_half(h[0][t]));
           }
           for (int e = 0; e < 2; e++)
-            out[((((size_t)s * L.nt + tl) * mats + q) * 2 + e) * 64 + l] =
+            out[((((size_t)s * L.nt + tl) * 2 + q) * 2 + e) * 64 + l] =
                 make_uint4(h[e][0] | (uint32_t)h[e][1] << 16, h[e][2] | (uint32_t)h[e][3] << 16,
                            h[e][4] | (uint32_t)h[e][5] << 16, h[e][6] | (uint32_t)h[e][7] << 16);
         }
 }
 }  // namespace
 
-size_t orbit_gen_box_floats(int p, int hh) { return gen_size(p, hh, 0); }
-size_t orbit_gen_frags(int p, int hh) { return gen_size(p, hh, 1); }
-size_t orbit_gen_rows(int p, int hh) { return gen_size(p, hh, 2); }
+size_t orbit_gen_box_floats(int p) { return gen_size(p, 0); }
+size_t orbit_gen_frags(int p) { return gen_size(p, 1); }
+size_t orbit_gen_rows(int p) { return gen_size(p, 2); }
 
 void orbit_gen_fragments(const double* C, const double* S, int ld, int p, int sa_e, uint4* out) {
   switch (p) {

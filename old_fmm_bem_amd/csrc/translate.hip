@@ -285,26 +285,22 @@ int Engine::run_m2m(int lev) {
   if (hh) {
     return dispatch_hp(p, [&](auto pc) -> int {
       constexpr int P = decltype(pc)::value, V = 2 * MLayout<P>::VS;
-      {
-        k_translate<V, double, 0><<<grid, TR_NT, 0, stream>>>(
-            nbp, sj.cfirst[lev].as<int>(), sj.bkey[lev + 1].as<uint32_t>(), nullptr, nullptr, nullptr,
-            mexp[lev + 1].as<double>(), m2m_part.as<double>(), m2m_ops<double>(lev));
-        k_m2l_reduce<double><<<(int)((n + 255) / 256), 256, 0, stream>>>(n, 8, m2m_part.as<double>(),
-                                                                         mexp[lev].as<double>(), 1);
-      }
+      k_translate<V, double, 0><<<grid, TR_NT, 0, stream>>>(
+          nbp, sj.cfirst[lev].as<int>(), sj.bkey[lev + 1].as<uint32_t>(), nullptr, nullptr, nullptr,
+          mexp[lev + 1].as<double>(), m2m_part.as<double>(), m2m_ops<double>(lev));
+      k_m2l_reduce<double><<<(int)((n + 255) / 256), 256, 0, stream>>>(n, 8, m2m_part.as<double>(),
+                                                                       mexp[lev].as<double>(), 1);
       FMMX_HIP(hipGetLastError());
       return FMMX_OK;
     });
   }
   auto m2m = [&](auto pc) -> int {
     constexpr int P = decltype(pc)::value, V = MLayout<P>::VS;
-    {
-      k_translate<V, double, 0><<<grid, TR_NT, 0, stream>>>(
-          nbp, sj.cfirst[lev].as<int>(), sj.bkey[lev + 1].as<uint32_t>(), nullptr, nullptr, nullptr,
-          mexp[lev + 1].as<double>(), m2m_part.as<double>(), m2m_ops<double>(lev));
-      k_m2l_reduce<double><<<(int)((n + 255) / 256), 256, 0, stream>>>(n, 8, m2m_part.as<double>(),
-                                                                       mexp[lev].as<double>(), 1);
-    }
+    k_translate<V, double, 0><<<grid, TR_NT, 0, stream>>>(
+        nbp, sj.cfirst[lev].as<int>(), sj.bkey[lev + 1].as<uint32_t>(), nullptr, nullptr, nullptr,
+        mexp[lev + 1].as<double>(), m2m_part.as<double>(), m2m_ops<double>(lev));
+    k_m2l_reduce<double><<<(int)((n + 255) / 256), 256, 0, stream>>>(n, 8, m2m_part.as<double>(),
+                                                                     mexp[lev].as<double>(), 1);
     FMMX_HIP(hipGetLastError());
     return FMMX_OK;
   };
