@@ -314,6 +314,20 @@ def main():
         # orders that has; else the leaf level on vector FMA) on the FP64 peak
         # (matrix = vector)
         all64 = bool(st64["m2l_all_levels"])
+        if all64:
+            # executed MFMA work per pair: 63 products for 189 pairs, each of tiles of 16 rows
+            # by k-steps of 4 slots of a class, eight per octet; the last octet of the larger
+            # classes ends with its last word that any has
+            size = [0] * 8
+            for n in range(a.p):
+                for m in range(n + 1):
+                    for im in range(2 if m else 1):
+                        size[((m ^ im) & 1) | im << 1 | ((n + m) & 1) << 2] += 1
+            no = 0
+            while sum(c > 4 * no for c in size) > 4 or max(size) > 4 * no + 8:
+                no += 1
+            nks = 8 * no + (0 if max(size) <= 4 * no else 8 if max(size) > 4 * no + 4 else 4)
+            exec64 = 63 / 189 * 2.0 * 16 * sum((c + 15) // 16 for c in size) * 4 * nks
         fl64 = 2.0 * a.p ** 4 * st64["m2l_pairs" if all64 else "m2l_pairs_leaf"]
         ach64 = fl64 / (ph64["ms_m2l_leaf"] * 1e-3) / 1e12
         fp64["roofline"] = {"bound": "mfma" if all64 else "valu", "achieved": ach64, "peak": PEAK["fp64_vector"], "unit": "TFLOP/s",
@@ -321,6 +335,8 @@ def main():
                             "kernel": f"k_m2l_of<{a.p}>, levels 2-{lmax} in one launch" if all64
                             else f"k_m2l_vec<{a.p}, double>, leaf level",
                             "ms_per_launch": ph64["ms_m2l_leaf"]}
+        if all64:
+            fp64["roofline"]["executed_flop_per_algorithmic"] = exec64 / (2.0 * a.p ** 4)
         f64.close()
 
     # dominant kernel and its roofline position.  The M2L launch (one launch

@@ -66,9 +66,10 @@ constexpr int ORB_NTH = 64 * ORB_WPG, ORB_TN = 16 * ORB_WPG;
 // product later, copied global -> LDS without registers.
 //
 // What bounds it (N = 1M, p = 10, levels 2-5): the vector units (transform,
-// split, addresses; 8e7 instructions, 0.14 ms), the LDS reads of the fragments
-// and the L1 accesses of the gather (0.14 ms each) and the MFMAs (0.09 ms)
-// have to overlap, and a workgroup's waves move from step to step together.
+// split, addresses; 6.9e7 instructions, 0.11 ms), the LDS accesses (0.14 ms), the
+// L1 accesses of the gather and the MFMAs (0.09 ms) have to overlap, and a
+// workgroup's waves move from step to step together: by the counters none is busy
+// for half of the launch.
 // 0.331 ms for the launch with two workgroups on a CU (128 registers, 76 KB of
 // LDS), 0.42 with one (162 registers; holding the fragments of 2 row classes
 // instead of 1 spills, 0.357).  Words loaded straight in the product's lane

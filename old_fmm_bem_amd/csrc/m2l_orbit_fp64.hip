@@ -55,8 +55,9 @@ constexpr int F64_NTH = 64 * ORB_WPG, F64_TN = 16 * ORB_WPG;
 // buffers of eight k-steps, copied one step ahead; one barrier per step.
 //
 // What bounds it: the FP64 matrix cores (64 cycles per MFMA at the 78.6
-// TFLOP/s of the card), on row tiles padded to 16: 224 MFMAs per product and 16
-// targets at p = 10, where 100 x 100 are 156.  N = 250k, p = 10,
+// TFLOP/s of the card; busy for 49 % of the launch below by the counters, the LDS
+// for 16 %) and the steps' barriers, on row tiles padded to 16: 224 MFMAs per
+// product and 16 targets at p = 10, where 100 x 100 are 156.  N = 250k, p = 10,
 // lmax 4 (640,584 pairs): 0.228 ms for the launch of all levels, beside the near
 // field; 0.89 + 1.34 ms as 189 products per target on the vector units with
 // operands re-read from LDS, which this replaces.

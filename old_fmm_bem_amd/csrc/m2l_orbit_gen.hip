@@ -101,10 +101,11 @@ constexpr int GEN_NTH = 64 * ORB_WPG, GEN_TN = 16 * ORB_WPG;
 // fragments (48 KB at P = 12): the next step's are copied while this one's
 // products run (144 MFMAs per wave), one barrier per step.
 //
-// What bounds it: waves without a source at an offset wait for the others of
-// their workgroup, so on a surface a SIMD often has one wave to hide the LDS
-// latency behind.  Sphere of 1M points, p = 12, lmax 6 (levels 2-6, 1.12M
-// pairs): 1.39 ms for the launch, 8.87 ms as FP32 MFMA products of 288 x 288
+// What bounds it: latency.  By the counters (sphere of 1M points, p = 12) the
+// matrix cores are busy for 29 % of the launch, the LDS for 30 %, the vector units
+// for 15 %: one workgroup per CU, whose two waves per SIMD move behind a barrier per
+// step, and for 27 % of the CU time none.  Levels 2-6 there (1.12M pairs): 1.35 ms
+// for the launch, 8.87 ms as FP32 MFMA products of 288 x 288
 // operators per offset, which this replaces (1.64 ms with each tile's fragments
 // waited for before its products).  Taking products without any source in the
 // workgroup off its list beforehand gained nothing: few are empty for 128
