@@ -514,7 +514,10 @@ void Engine::drop_graph() {
   if (graph) (void)hipGraphDestroy(graph);
   gexec = nullptr;
   graph = nullptr;
-  if (!kept.empty()) (void)hipDeviceSynchronize();
+  if (!kept.empty()) {
+    (void)hipSetDevice(device);
+    (void)hipDeviceSynchronize();
+  }
   for (void* b : kept) (void)hipFree(b);
   kept.clear();
 }
